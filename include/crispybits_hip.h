@@ -153,6 +153,16 @@ int cbk_packed_gemm(const void* x, int dtype, int64_t M, int64_t K,
                     int64_t N, int bits, int group_size, int act, int use_matrix_cores,
                     void* out, int device, void* stream);
 
+/* The same calls with a partial buffer, which lets a GEMM of few tiles split K over the idle
+ * CUs (additive; no counterpart in the reference).  cbk_gemm_partial_floats: the fp32
+ * elements `partial` must hold (0: the call needs none; gate_up: the gate-up GEMM's).  A call
+ * without a large enough buffer runs unsplit: same result up to the order of the fp32 sums. */
+int64_t cbk_gemm_partial_floats(int dtype, int64_t M, int64_t N, int64_t K, int gate_up);
+int cbk_packed_gemm_ws(const void* x, int dtype, int64_t M, int64_t K,
+                       const int32_t* packed, const void* scales, const void* zeros, const void* bias,
+                       int64_t N, int bits, int group_size, int act, int use_matrix_cores,
+                       float* partial, int64_t partial_floats, void* out, int device, void* stream);
+
 /* Prefill gate-up: out[M,N] = RN_T(RN_T(silu(x . G-hat^T)) * RN_T(x . U-hat^T)) in one launch,
  * bit-identical to two cbk_packed_gemm calls (the gate's with act = 2) followed by an
  * elementwise product in T.  No counterpart in the reference's _C: it replaces the
@@ -164,6 +174,29 @@ int cbk_packed_gemm_gate_up(const void* x, int dtype, int64_t M, int64_t K,
                             const int32_t* packed_gate, const void* scales_gate, const void* zeros_gate,
                             const int32_t* packed_up, const void* scales_up, const void* zeros_up,
                             int64_t N, int bits, int group_size, void* out, int device, void* stream);
+int cbk_packed_gemm_gate_up_ws(const void* x, int dtype, int64_t M, int64_t K,
+                               const int32_t* packed_gate, const void* scales_gate, const void* zeros_gate,
+                               const int32_t* packed_up, const void* scales_up, const void* zeros_up,
+                               int64_t N, int bits, int group_size, float* partial, int64_t partial_floats,
+                               void* out, int device, void* stream);
+
+/* Prefill Q, K and V in one launch (additive; it replaces the three GEMMs, the column restore and
+ * the rotation of the reference's ops.fused_qkv above the decode threshold, ops.py:248-273).
+ * perm_hd > 0: Q and K are stored pair-interleaved per head of perm_hd rows and come out in the
+ * original column order, rotated when rope_cos / rope_sin [M, perm_hd] are given (in fp32 when
+ * rope_f32, else in x's dtype): each value rounded to T as its GEMM stores it, rotated in fp32 and
+ * rounded once.  Widths may differ.  fp16 / bf16 x only, with K % 8 == 0 and 16-byte aligned x,
+ * packed, scales and zeros; other calls return CBK_ENOTSUP (nothing launched).
+ * cbk_gemm_qkv_partial_floats: the fp32 elements `partial` must hold for K splits (0: none). */
+int64_t cbk_gemm_qkv_partial_floats(int dtype, int64_t M, int64_t nq, int64_t nk, int64_t nv, int64_t K);
+int cbk_packed_gemm_qkv(const void* x, int dtype, int64_t M, int64_t K,
+                        const int32_t* wq, const void* sq, const void* zq, const void* bq, int64_t nq,
+                        const int32_t* wk, const void* sk, const void* zk, const void* bk, int64_t nk,
+                        const int32_t* wv, const void* sv, const void* zv, const void* bv, int64_t nv,
+                        const void* rope_cos, const void* rope_sin, int rope_f32, int perm_hd,
+                        int bits_q, int bits_k, int bits_v, int group_size, float* partial,
+                        int64_t partial_floats, void* out_q, void* out_k, void* out_v,
+                        int device, void* stream);
 
 /* Format producer on the device: group-affine quantization of w[N,K] (fp16 / bf16 /
  * fp32) to `bits`-bit codes, packed as the kernels read them, with fp16 / bf16 / fp32

@@ -335,13 +335,24 @@ def fused_gate_up(x: torch.Tensor, gate: PackedLinearWeight, up: PackedLinearWei
     return _restore(y, lead)
 
 
+def _prefill_qkv(x2, q, k, v, cos2, sin2):
+    """Q, K and V of a prefill batch in one launch, or None where the backend has no such launch
+    for the call."""
+    if not hasattr(_C, "packed_gemm_qkv"):
+        return None
+    return _C.packed_gemm_qkv(x2, q.packed, q.scales, q.zeros, q.bias, k.packed, k.scales, k.zeros, k.bias, v.packed,
+                              v.scales, v.zeros, v.bias, cos2, sin2, q.rope_perm_head_dim, (q.bits, k.bits, v.bits),
+                              q.in_features, q.group_size)
+
+
 def fused_qkv(x: torch.Tensor, q: PackedLinearWeight, k: PackedLinearWeight, v: PackedLinearWeight,
               split_k: Optional[int] = None, rho: int = 1,
               rope: Optional[Tuple[torch.Tensor, torch.Tensor, int]] = None,
               decode_threshold: int = DECODE_THRESHOLD, workspace: Optional[torch.Tensor] = None):
     """Q, K and V of one attention layer.  Decode: one kernel (GQA widths, biases, and with
     ``rope=(cos, sin, head_dim)`` HF rotate-half RoPE on Q/K stored pair-interleaved).
-    Prefill: three GEMMs, then RoPE on the stored layout and the original column order."""
+    Prefill: one GEMM launch over the three projections' tiles that ends in the same (fp16 / bf16
+    activations), else three GEMMs, then RoPE on the stored layout and the original column order."""
     _check_ext()
     if not (q.in_features == k.in_features == v.in_features and q.group_size == k.group_size == v.group_size):
         raise ValueError("Q/K/V must share in_features and group_size")
@@ -370,14 +381,16 @@ def fused_qkv(x: torch.Tensor, q: PackedLinearWeight, k: PackedLinearWeight, v: 
                             v.packed, v.scales, v.zeros, v.bias, rc, rs, head_dim, perm, bits, q.in_features,
                             q.group_size, pk, rho, workspace)
     else:
-        outs = []
-        for i, w in enumerate((q, k, v)):
-            y = _linear(x2, w, None, 1, 0, 0, None, True)
-            if i < 2 and cos2 is not None:
-                y = _rope_stored(y, cos2, sin2, head_dim)
-            elif w.rope_perm_head_dim:
-                y = _original_columns(y, w.rope_perm_head_dim)
-            outs.append(y)
+        outs = _prefill_qkv(x2, q, k, v, cos2, sin2)
+        if outs is None:
+            outs = []
+            for i, w in enumerate((q, k, v)):
+                y = _linear(x2, w, None, 1, 0, 0, None, True)
+                if i < 2 and cos2 is not None:
+                    y = _rope_stored(y, cos2, sin2, head_dim)
+                elif w.rope_perm_head_dim:
+                    y = _original_columns(y, w.rope_perm_head_dim)
+                outs.append(y)
     return tuple(_restore(o, lead) for o in outs)
 
 

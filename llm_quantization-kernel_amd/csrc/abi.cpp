@@ -701,6 +701,27 @@ int qkv_common(const void* x, int dtype, int64_t M, int64_t K, const int32_t* wq
     return run_decode(A, dtype, CBK_MODE_QKV, mixed, split_k, rho, partial, device, stream);
 }
 
+// The plan of a 16-bit matrix-core GEMM over `ntiles` column tiles, with its split fields set in
+// A.  K splits need the caller's partial buffer; without one the call runs unsplit.  Without a
+// counter window (split_window) a combine launch adds the partials, in the same order.
+GemmPlan plan_gemm_f16(GemmArgs& A, int64_t ntiles, float* partial, int64_t partial_floats, int device,
+                       hipStream_t s) {
+    GemmPlan p = gemm_f16_plan(A.M, ntiles, A.K, true);
+    if (p.S > 1 && (!partial || partial_floats < p.partial_floats)) p = gemm_f16_plan(A.M, ntiles, A.K, false);
+    A.S = p.S;
+    A.partial = p.S > 1 ? partial : nullptr;
+    A.split_cnt = p.S > 1 && p.tiles <= SPLIT_COUNTERS ? split_window(device, s) : nullptr;
+    return p;
+}
+
+int run_gemm_f16(GemmArgs& A, int dtype, int mode, float* partial, int64_t partial_floats, int device,
+                 hipStream_t s, const char* what) {
+    const GemmPlan p =
+        plan_gemm_f16(A, gemm_f16_ntiles(A.N, mode == GEMM_GATEUP), partial, partial_floats, device, s);
+    const hipError_t e = launch_gemm_f16(A, dtype, p, s, mode);
+    return e == hipSuccess ? CBK_OK : hip_fail(e, what);
+}
+
 }  // namespace
 
 namespace cbk {
@@ -899,6 +920,19 @@ int cbk_fused_qkv_mixed(const void* x, int dtype, int64_t M, int64_t K, const in
 int cbk_packed_gemm(const void* x, int dtype, int64_t M, int64_t K, const int32_t* packed, const void* scales,
                     const void* zeros, const void* bias, int64_t N, int bits, int group_size, int act,
                     int use_matrix_cores, void* out, int device, void* stream) {
+    return cbk_packed_gemm_ws(x, dtype, M, K, packed, scales, zeros, bias, N, bits, group_size, act,
+                              use_matrix_cores, nullptr, 0, out, device, stream);
+}
+
+int64_t cbk_gemm_partial_floats(int dtype, int64_t M, int64_t N, int64_t K, int gate_up) {
+    if ((dtype != CBK_F16 && dtype != CBK_BF16) || M <= 0 || N <= 0 || K <= 0) return 0;
+    return gemm_f16_plan(M, gemm_f16_ntiles(N, gate_up != 0), K, true).partial_floats;
+}
+
+int cbk_packed_gemm_ws(const void* x, int dtype, int64_t M, int64_t K, const int32_t* packed, const void* scales,
+                       const void* zeros, const void* bias, int64_t N, int bits, int group_size, int act,
+                       int use_matrix_cores, float* partial, int64_t partial_floats, void* out, int device,
+                       void* stream) {
     int rc = check_x(x, dtype, M, K);
     if (rc) return rc;
     if ((rc = check_weight(packed, scales, zeros, N, bits, group_size, "packed_gemm"))) return rc;
@@ -927,9 +961,9 @@ int cbk_packed_gemm(const void* x, int dtype, int64_t M, int64_t K, const int32_
     A.divG = make_fastdiv((uint32_t)group_size);
     A.xvec = (K % 8 == 0) && (reinterpret_cast<uintptr_t>(x) % 16 == 0);
     const bool mc = use_matrix_cores && (dtype == CBK_F16 || dtype == CBK_BF16);
-    hipError_t e;
-    if (mc && gemm_f16_supported(A)) e = launch_gemm_f16(A, dtype, s);
-    else e = mc ? launch_gemm_mfma(A, dtype, s) : launch_gemm_f32(A, dtype, s);
+    if (mc && gemm_f16_supported(A))
+        return run_gemm_f16(A, dtype, GEMM_PLAIN, partial, partial_floats, device, s, "packed_gemm: launch");
+    const hipError_t e = mc ? launch_gemm_mfma(A, dtype, s) : launch_gemm_f32(A, dtype, s);
     if (e != hipSuccess) return hip_fail(e, "packed_gemm: launch");
     return CBK_OK;
 }
@@ -938,6 +972,14 @@ int cbk_packed_gemm_gate_up(const void* x, int dtype, int64_t M, int64_t K, cons
                             const void* scales_gate, const void* zeros_gate, const int32_t* packed_up,
                             const void* scales_up, const void* zeros_up, int64_t N, int bits, int group_size,
                             void* out, int device, void* stream) {
+    return cbk_packed_gemm_gate_up_ws(x, dtype, M, K, packed_gate, scales_gate, zeros_gate, packed_up, scales_up,
+                                      zeros_up, N, bits, group_size, nullptr, 0, out, device, stream);
+}
+
+int cbk_packed_gemm_gate_up_ws(const void* x, int dtype, int64_t M, int64_t K, const int32_t* packed_gate,
+                               const void* scales_gate, const void* zeros_gate, const int32_t* packed_up,
+                               const void* scales_up, const void* zeros_up, int64_t N, int bits, int group_size,
+                               float* partial, int64_t partial_floats, void* out, int device, void* stream) {
     int rc = check_x(x, dtype, M, K);
     if (rc) return rc;
     if ((rc = check_weight(packed_gate, scales_gate, zeros_gate, N, bits, group_size, "packed_gemm_gate_up(gate)")))
@@ -973,9 +1015,82 @@ int cbk_packed_gemm_gate_up(const void* x, int dtype, int64_t M, int64_t K, cons
     if (M == 0) return CBK_OK;
     DeviceGuard guard(device);
     if (guard.err != hipSuccess) return hip_fail(guard.err, "set device");
-    const hipError_t e = launch_gemm_f16(A, dtype, reinterpret_cast<hipStream_t>(stream), true);
-    if (e != hipSuccess) return hip_fail(e, "packed_gemm_gate_up: launch");
-    return CBK_OK;
+    return run_gemm_f16(A, dtype, GEMM_GATEUP, partial, partial_floats, device, reinterpret_cast<hipStream_t>(stream),
+                        "packed_gemm_gate_up: launch");
+}
+
+int64_t cbk_gemm_qkv_partial_floats(int dtype, int64_t M, int64_t nq, int64_t nk, int64_t nv, int64_t K) {
+    if ((dtype != CBK_F16 && dtype != CBK_BF16) || M <= 0 || nq <= 0 || nk <= 0 || nv <= 0 || K <= 0) return 0;
+    const int64_t nt = gemm_f16_ntiles(nq, false) + gemm_f16_ntiles(nk, false) + gemm_f16_ntiles(nv, false);
+    return gemm_f16_plan(M, nt, K, true).partial_floats;
+}
+
+int cbk_packed_gemm_qkv(const void* x, int dtype, int64_t M, int64_t K, const int32_t* wq, const void* sq,
+                        const void* zq, const void* bq, int64_t nq, const int32_t* wk, const void* sk, const void* zk,
+                        const void* bk, int64_t nk, const int32_t* wv, const void* sv, const void* zv, const void* bv,
+                        int64_t nv, const void* rope_cos, const void* rope_sin, int rope_f32, int perm_hd, int bits_q,
+                        int bits_k, int bits_v, int group_size, float* partial, int64_t partial_floats, void* out_q,
+                        void* out_k, void* out_v, int device, void* stream) {
+    int rc = check_x(x, dtype, M, K);
+    if (rc) return rc;
+    if ((rc = check_weight(wq, sq, zq, nq, bits_q, group_size, "packed_gemm_qkv(q)"))) return rc;
+    if ((rc = check_weight(wk, sk, zk, nk, bits_k, group_size, "packed_gemm_qkv(k)"))) return rc;
+    if ((rc = check_weight(wv, sv, zv, nv, bits_v, group_size, "packed_gemm_qkv(v)"))) return rc;
+    if (!out_q || !out_k || !out_v) return fail(CBK_EINVAL, "packed_gemm_qkv: outputs must be non-null");
+    if (perm_hd < 0) return fail(CBK_EINVAL, "head_dim must be >= 0");
+    if (perm_hd > 0) {
+        if (perm_hd % 2) return fail(CBK_EINVAL, "perm head_dim must be even");
+        if (nq % perm_hd || nk % perm_hd) return fail(CBK_EINVAL, "Q/K widths must be multiples of head_dim");
+    }
+    if ((rope_cos != nullptr) != (rope_sin != nullptr)) return fail(CBK_EINVAL, "cos/sin shape mismatch");
+    if (rope_cos && perm_hd == 0)
+        return fail(CBK_EINVAL, "fused RoPE needs Q/K weights stored pair-interleaved with the same head_dim");
+    if (dtype != CBK_F16 && dtype != CBK_BF16)
+        return fail(CBK_ENOTSUP, "packed_gemm_qkv: x must be fp16 or bf16 (the 16-bit matrix cores)");
+    GemmQkvArgs Q{};
+    GemmArgs& A = Q.a;
+    A.x = x;
+    A.M = (int)M;
+    A.K = (int)K;
+    A.C = (int)ceil_div(K, 32);
+    A.G = (int)ceil_div(K, group_size);
+    A.gs = group_size;
+    A.act = ACT_NONE;
+    A.divG = make_fastdiv((uint32_t)group_size);
+    A.rope_cos = rope_cos;
+    A.rope_sin = rope_sin;
+    A.rope_f32 = rope_f32;
+    A.perm_hd = perm_hd;
+    A.divHD = make_fastdiv((uint32_t)std::max(perm_hd, 1));
+    const int32_t* w[3] = {wq, wk, wv};
+    const void *s[3] = {sq, sk, sv}, *z[3] = {zq, zk, zv}, *b[3] = {bq, bk, bv};
+    void* out[3] = {out_q, out_k, out_v};
+    const int64_t n[3] = {nq, nk, nv};
+    const int bits[3] = {bits_q, bits_k, bits_v};
+    int64_t ntiles = 0;
+    for (int i = 0; i < 3; ++i) {
+        A.w = Q.w[i] = reinterpret_cast<const uint32_t*>(w[i]);
+        A.s = Q.s[i] = s[i];
+        A.z = Q.z[i] = z[i];
+        Q.b[i] = b[i];
+        Q.out[i] = out[i];
+        A.N = Q.n[i] = (int)n[i];
+        Q.bits[i] = bits[i];
+        A.wpr = A.C * bits[i];
+        if (!gemm_f16_supported(A))
+            return fail(CBK_ENOTSUP, "packed_gemm_qkv: needs K %% 8 == 0 and 16-byte aligned x, packed, scales "
+                                     "and zeros");
+        ntiles += gemm_f16_ntiles(n[i], false);
+    }
+    if (ceil_div(std::max<int64_t>(M, 1), 32) * ntiles >= INT32_MAX / 32)
+        return fail(CBK_ENOTSUP, "packed_gemm_qkv: too many tiles for one launch");
+    if (M == 0) return CBK_OK;
+    DeviceGuard guard(device);
+    if (guard.err != hipSuccess) return hip_fail(guard.err, "set device");
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    const GemmPlan p = plan_gemm_f16(A, ntiles, partial, partial_floats, device, st);
+    const hipError_t e = launch_gemm_f16_qkv(Q, dtype, p, st);
+    return e == hipSuccess ? CBK_OK : hip_fail(e, "packed_gemm_qkv: launch");
 }
 
 int cbk_quantize_pack(const void* w, int dtype, int64_t N, int64_t K, int bits, int group_size, int scheme,

@@ -306,21 +306,24 @@ __device__ __forceinline__ void put_unit(const GemvArgs& A, int p, int b, int v0
     if (two) partial_put(row + v0 + 1, y1);
 }
 
-// After the workgroup's partial_put calls: returns, in every thread, whether this
-// workgroup combines row block `blk`.  `flag` is a word of LDS that no thread reads or
-// writes across this call.
-__device__ __forceinline__ bool split_arrive(const GemvArgs& A, int blk, int* flag) {
+// After the workgroup's partial stores: returns, in every thread, whether this workgroup
+// (the last of `parts` to count itself in at `c`) combines the block.  `flag` is a word of
+// LDS that no thread reads or writes across this call.
+__device__ __forceinline__ bool split_arrive(uint32_t* c, int parts, int* flag) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this wave's partials are stored
     __syncthreads();
     if (threadIdx.x == 0) {
-        uint32_t* c = A.split_cnt + blk;
         const uint32_t old = __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const bool last = old + 1u == (uint32_t)A.P;
+        const bool last = old + 1u == (uint32_t)parts;
         if (last) __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         *flag = last ? 1 : 0;
     }
     __syncthreads();
     return *flag != 0;
+}
+
+__device__ __forceinline__ bool split_arrive(const GemvArgs& A, int blk, int* flag) {
+    return split_arrive(A.split_cnt + blk, A.P, flag);
 }
 
 // The finish unit starting at v0 of batch row b summed over splits 0 .. P - 1 in that

@@ -49,10 +49,33 @@ struct GemmArgs {
     int M, N, K, C, G, gs, wpr, bits, act;
     int xvec;               // x is 16-byte aligned and K % 8 == 0 (vector activation loads)
     FastDiv divG;           // by the group size
+    // 16-bit matrix-core GEMM: K splits per tile, their partial tiles, an arrival counter per tile
+    int S;
+    float* partial;
+    uint32_t* split_cnt;
     const uint32_t* w2;     // gate-up GEMM: the up projection's packed [N, wpr], scales, zeros
     const void* s2;
     const void* z2;
+    // fused QKV: Q and K stored pair-interleaved per head of perm_hd rows (0: in order), the
+    // RoPE tables [M, perm_hd] (nullptr: none) in fp32 or the activations' dtype
+    const void* rope_cos;
+    const void* rope_sin;
+    int perm_hd, rope_f32;
+    FastDiv divHD;          // by perm_hd
 };
+
+// The fused-QKV GEMM: a's fields common to the three projections, and each one's own.
+struct GemmQkvArgs {
+    GemmArgs a;
+    const uint32_t* w[3];
+    const void* s[3];
+    const void* z[3];
+    const void* b[3];
+    void* out[3];
+    int n[3], bits[3];
+    int first[3];           // each projection's first tile
+};
+enum { GEMM_PLAIN = 0, GEMM_GATEUP = 1, GEMM_QKV = 2 };
 
 // gemm.hip: fp16 / bf16 on the 16-bit matrix cores, any alignment.
 hipError_t launch_gemm_mfma(const GemmArgs& A, int dt, hipStream_t stream);
@@ -62,8 +85,31 @@ hipError_t launch_gemm_f32(const GemmArgs& A, int dt, hipStream_t stream);
 
 // gemm_f16.hip: fp16 or bf16 (dt), K % 8 == 0, 16-byte aligned x.  gate_up: out =
 // silu(x . W-hat^T) * (x . W2-hat^T), each factor rounded to the dtype first (no bias).
+// A call's plan: tiles of 32 mb rows (mb 1, 2 or 4) x 128 columns, S K splits each.
+struct GemmPlan {
+    int mb = 4, S = 1;
+    int64_t tiles = 0, partial_floats = 0;       // tiles, and the fp32 partial tiles of S > 1
+};
+// ntiles: 128-column tiles over all projections (64 output pairs a tile for gate-up); split: K
+// splits allowed.
+GemmPlan gemm_f16_plan(int64_t M, int64_t ntiles, int64_t K, bool split);
+inline int64_t gemm_f16_ntiles(int64_t N, bool gate_up) { return gate_up ? (N + 63) / 64 : (N + 127) / 128; }
 bool gemm_f16_supported(const GemmArgs& A);
-hipError_t launch_gemm_f16(const GemmArgs& A, int dt, hipStream_t stream, bool gate_up = false);
+// A.S, A.partial and A.split_cnt set when the plan has splits (S = 1 otherwise); without counters
+// a combine launch follows.  mode: GEMM_PLAIN or GEMM_GATEUP.
+hipError_t launch_gemm_f16(const GemmArgs& A, int dt, const GemmPlan& plan, hipStream_t stream, int mode);
+hipError_t launch_gemm_f16_qkv(GemmQkvArgs& Q, int dt, const GemmPlan& plan, hipStream_t stream);
+
+// The kernels of a tile height, one translation unit each (gemm_f16_mb*.hip).
+struct GemmKernel {
+    const void* f = nullptr;
+    const void* combine = nullptr;
+    int lds = 0, combine_lds = 0;
+};
+GemmKernel gemm_f16_mb1(int dt, int bits, bool tail, bool gs128, int mode);
+GemmKernel gemm_f16_mb2(int dt, int bits, bool tail, bool gs128, int mode);
+GemmKernel gemm_f16_mb4(int dt, int bits, bool tail, bool gs128, int mode);
+GemmKernel gemm_f16_mb4s(int dt, int bits, bool tail, bool gs128, int mode);   // with K splits
 
 // quant.hip: group-affine quantizer + bit packer (the format's producer).
 struct QuantArgs {

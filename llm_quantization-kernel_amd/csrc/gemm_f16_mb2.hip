@@ -1,0 +1,10 @@
+// gemm_f16_mb2.hip -- the fp16 / bf16 prefill GEMM (gemm_f16_tile.hpp) with 64-row tiles (K split or not).
+#include "gemm_f16_tile.hpp"
+
+namespace cbk {
+
+GemmKernel gemm_f16_mb2(int dt, int bits, bool tail, bool gs128, int mode) {
+    return kernel_of<2, true>(dt, bits, tail, gs128, mode);
+}
+
+}  // namespace cbk

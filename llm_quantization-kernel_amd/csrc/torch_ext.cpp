@@ -121,6 +121,14 @@ Tensor partial_for(const Tensor& x, int64_t M, int64_t V, int64_t K, int64_t gs,
     return n > 0 ? at::empty({n}, x.options().dtype(at::kFloat)) : Tensor();
 }
 
+// Partial tiles of a prefill GEMM with K splits (undefined when its plan has none).
+Tensor gemm_partial(const Tensor& x, int64_t N, bool gate_up) {
+    const int64_t n = cbk_gemm_partial_floats(dtype_of(x.scalar_type()), x.size(0), N, x.size(1), gate_up ? 1 : 0);
+    return n > 0 ? at::empty({n}, x.options().dtype(at::kFloat)) : Tensor();
+}
+
+int64_t numel_of(const Tensor& t) { return t.defined() ? t.numel() : 0; }
+
 void* tensor_ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 
 // ------------------------------------------------------------------------------------- ops
@@ -155,9 +163,11 @@ Tensor packed_gemm(const Tensor& x, const Tensor& packed, const Tensor& scales, 
     Tensor out = at::empty({M, N}, x.options());
     if (M == 0) return out;
     const int dev = x.get_device();
-    ok(cbk_packed_gemm(x.data_ptr(), dtype_of(x.scalar_type()), M, in_features, packed.data_ptr<int32_t>(),
-                       scales.data_ptr(), zeros.data_ptr(), b, N, (int)bits, (int)group_size, (int)act,
-                       use_tensor_cores ? 1 : 0, out.data_ptr(), dev, stream_of(dev)));
+    const Tensor part = use_tensor_cores ? gemm_partial(x, N, false) : Tensor();
+    ok(cbk_packed_gemm_ws(x.data_ptr(), dtype_of(x.scalar_type()), M, in_features, packed.data_ptr<int32_t>(),
+                          scales.data_ptr(), zeros.data_ptr(), b, N, (int)bits, (int)group_size, (int)act,
+                          use_tensor_cores ? 1 : 0, static_cast<float*>(tensor_ptr(part)), numel_of(part),
+                          out.data_ptr(), dev, stream_of(dev)));
     return out;
 }
 
@@ -195,10 +205,12 @@ Tensor packed_gemm_gate_up(const Tensor& x, const Tensor& wg, const Tensor& sg, 
     Tensor out = at::empty({M, N}, x.options());
     if (M == 0) return out;
     const int dev = x.get_device();
-    const int rc = cbk_packed_gemm_gate_up(x.data_ptr(), dtype_of(x.scalar_type()), M, in_features,
-                                           wg.data_ptr<int32_t>(), sg.data_ptr(), zg.data_ptr(),
-                                           wu.data_ptr<int32_t>(), su.data_ptr(), zu.data_ptr(), N, (int)bits,
-                                           (int)group_size, out.data_ptr(), dev, stream_of(dev));
+    const Tensor part = gemm_partial(x, N, true);
+    const int rc = cbk_packed_gemm_gate_up_ws(x.data_ptr(), dtype_of(x.scalar_type()), M, in_features,
+                                              wg.data_ptr<int32_t>(), sg.data_ptr(), zg.data_ptr(),
+                                              wu.data_ptr<int32_t>(), su.data_ptr(), zu.data_ptr(), N, (int)bits,
+                                              (int)group_size, static_cast<float*>(tensor_ptr(part)),
+                                              numel_of(part), out.data_ptr(), dev, stream_of(dev));
     if (rc != CBK_ENOTSUP) {
         ok(rc);
         return out;
@@ -282,6 +294,52 @@ std::vector<Tensor> fused_qkv(const Tensor& x, const Tensor& wq, const Tensor& s
                                outs[2].data_ptr(), dev, stream_of(dev)));
     }
     return outs;
+}
+
+// Prefill Q, K and V in one launch; None for calls that launch does not take (fp32 or unaligned
+// x, RoPE tables in another dtype or on another device), which the caller runs as three GEMMs.
+// ``bits``: (q, k, v) widths.
+py::object packed_gemm_qkv(const Tensor& x, const Tensor& wq, const Tensor& sq, const Tensor& zq, const OptT& bq,
+                           const Tensor& wk, const Tensor& sk, const Tensor& zk, const OptT& bk, const Tensor& wv,
+                           const Tensor& sv, const Tensor& zv, const OptT& bv, const OptT& rope_cos,
+                           const OptT& rope_sin, int64_t perm_hd, std::tuple<int64_t, int64_t, int64_t> bits,
+                           int64_t in_features, int64_t group_size) {
+    const int64_t bw[3] = {std::get<0>(bits), std::get<1>(bits), std::get<2>(bits)};
+    check_x(x, in_features);
+    check_weight(x, wq, sq, zq, bw[0], in_features, group_size, "packed_gemm");
+    check_weight(x, wk, sk, zk, bw[1], in_features, group_size, "packed_gemm");
+    check_weight(x, wv, sv, zv, bw[2], in_features, group_size, "packed_gemm");
+    const int64_t nq = wq.size(0), nk = wk.size(0), nv = wv.size(0), M = x.size(0);
+    const void* pq = bias_ptr(bq, x, nq);
+    const void* pk = bias_ptr(bk, x, nk);
+    const void* pv = bias_ptr(bv, x, nv);
+    const at::ScalarType xt = x.scalar_type();
+    if (M == 0 || (xt != at::kHalf && xt != at::kBFloat16)) return py::none();
+    if (perm_hd < 0 || (perm_hd > 0 && (perm_hd % 2 || nq % perm_hd || nk % perm_hd))) return py::none();
+    Tensor rc, rs;
+    if (rope_cos.has_value()) {
+        const at::ScalarType t = rope_cos->scalar_type();
+        if (perm_hd == 0 || !rope_sin.has_value() || rope_sin->scalar_type() != t || (t != xt && t != at::kFloat) ||
+            rope_cos->device() != x.device() || rope_sin->device() != x.device() ||
+            rope_cos->numel() != M * perm_hd || rope_sin->numel() != M * perm_hd)
+            return py::none();
+        rc = rope_cos->contiguous();
+        rs = rope_sin->contiguous();
+    }
+    std::vector<Tensor> outs = {at::empty({M, nq}, x.options()), at::empty({M, nk}, x.options()),
+                                at::empty({M, nv}, x.options())};
+    const int64_t pf = cbk_gemm_qkv_partial_floats(dtype_of(xt), M, nq, nk, nv, in_features);
+    const Tensor part = pf > 0 ? at::empty({pf}, x.options().dtype(at::kFloat)) : Tensor();
+    const int dev = x.get_device();
+    const int r = cbk_packed_gemm_qkv(
+        x.data_ptr(), dtype_of(xt), M, in_features, wq.data_ptr<int32_t>(), sq.data_ptr(), zq.data_ptr(), pq, nq,
+        wk.data_ptr<int32_t>(), sk.data_ptr(), zk.data_ptr(), pk, nk, wv.data_ptr<int32_t>(), sv.data_ptr(),
+        zv.data_ptr(), pv, nv, tensor_ptr(rc), tensor_ptr(rs), rc.defined() && rc.scalar_type() == at::kFloat ? 1 : 0,
+        (int)perm_hd, (int)bw[0], (int)bw[1], (int)bw[2], (int)group_size, static_cast<float*>(tensor_ptr(part)), pf,
+        outs[0].data_ptr(), outs[1].data_ptr(), outs[2].data_ptr(), dev, stream_of(dev));
+    if (r == CBK_ENOTSUP) return py::none();
+    ok(r);
+    return py::cast(outs);
 }
 
 int current_device() { return c10::hip::current_device(); }
@@ -398,6 +456,8 @@ PYBIND11_MODULE(_ext, m) {
     m.def("packed_gemm_gate_up", &packed_gemm_gate_up,
           "Prefill gate-up: silu(x G^T) * (x U^T), one MFMA launch for fp16/bf16 x");
     m.def("fused_qkv", &fused_qkv, "Fused Q/K/V decode GEMV (GQA widths, biases, optional in-kernel RoPE)");
+    m.def("packed_gemm_qkv", &packed_gemm_qkv,
+          "Prefill Q, K and V (optional RoPE) in one MFMA launch for fp16/bf16 x, or None");
     m.def("sm_count", &sm_count, "Compute units of the current device");
     m.def("tile_n", &tile_n, "Virtual output rows per decode job tile (B_N of the underfill rule)");
     m.def("max_rho", &max_rho, "Occupancy-limited resident workgroups per CU", py::arg("bits"),

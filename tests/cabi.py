@@ -28,6 +28,13 @@ SIGS = {
                                  _P, _P, _P, _P, _L, _P, _P, _P, _P, _L, _P, _P, _P, _P, _L,
                                  _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _P]),
     "cbk_packed_gemm": (_I, [_P, _I, _L, _L, _P, _P, _P, _P, _L, _I, _I, _I, _I, _P, _I, _P]),
+    "cbk_gemm_qkv_partial_floats": (_L, [_I, _L, _L, _L, _L, _L]),
+    "cbk_packed_gemm_qkv": (_I, [_P, _I, _L, _L,
+                                 _P, _P, _P, _P, _L, _P, _P, _P, _P, _L, _P, _P, _P, _P, _L,
+                                 _P, _P, _I, _I, _I, _I, _I, _I, _P, _L, _P, _P, _P, _I, _P]),
+    "cbk_gemm_partial_floats": (_L, [_I, _L, _L, _L, _I]),
+    "cbk_packed_gemm_ws": (_I, [_P, _I, _L, _L, _P, _P, _P, _P, _L, _I, _I, _I, _I, _P, _L, _P, _I, _P]),
+    "cbk_packed_gemm_gate_up_ws": (_I, [_P, _I, _L, _L, _P, _P, _P, _P, _P, _P, _L, _I, _I, _P, _L, _P, _I, _P]),
     "cbk_packed_gemm_gate_up": (_I, [_P, _I, _L, _L, _P, _P, _P, _P, _P, _P, _L, _I, _I, _P, _I, _P]),
     "cbk_unpack_codes": (_I, [_P, _L, _L, _I, _P, _I, _P]),
     "cbk_quantize_pack": (_I, [_P, _I, _L, _L, _I, _I, _I, _P, _P, _P, _I, _I, _P]),

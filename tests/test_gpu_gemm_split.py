@@ -1,0 +1,125 @@
+"""The 16-bit prefill GEMM below a full chip: 32- and 64-row tiles, and K split over workgroups
+whose partial tiles are combined in the dispatch.
+
+The shapes have few tiles, so that the plan splits K (cbk_gemm_partial_floats > 0 says so), with
+splits that start inside a scale window, a ragged K in the last split, partial tiles in M and N, and
+zero points the packed-fp16 dequantization does not take.  The bar against the oracle is one output
+rounding (half an ulp, 2^-11 for fp16 and 2^-8 for bf16, of the largest output) plus the fp32 sums,
+K 2^-24 of the sum of magnitudes -- below 1e-4 of the largest output at these sizes."""
+import numpy as np
+import pytest
+import torch
+
+import cabi
+from crispybits_kernels import _C, fused_gate_up, ops, packed_linear
+from crispybits_kernels.io import from_packed_dict
+from crispybits_kernels.reference import pack_linear_dict
+from oracle import emulator as E
+
+pytestmark = pytest.mark.gpu
+
+BAR = {torch.float16: 2.0 ** -11 + 1e-4, torch.bfloat16: 2.0 ** -8 + 1e-4}
+CODE = {torch.float16: 0, torch.bfloat16: 1}
+
+
+def make(N, K, bits, dtype, gs, seed, bias=False, fractional=False):
+    g = torch.Generator().manual_seed(seed)
+    b = torch.randn(N, generator=g) if bias else None
+    d = pack_linear_dict(torch.randn(N, K, generator=g) * 0.05, bits, gs, b, dtype)
+    if fractional:
+        z = d["zeros"].clone()
+        z[: N // 2] += 0.375
+        d["zeros"] = z
+    W = E.gemm_weight64(d["packed"].numpy(), d["scales"].to(dtype).double().numpy(),
+                        d["zeros"].to(dtype).double().numpy(), bits, K, gs, dtype, True)
+    return from_packed_dict(d, "cuda", dtype), W, None if b is None else b.to(dtype).double().numpy()
+
+
+def randx(M, K, dtype, seed=3):
+    return torch.randn(M, K, generator=torch.Generator().manual_seed(seed)).to(dtype).cuda()
+
+
+def off(y, ref):
+    return float(np.abs(y.float().cpu().double().numpy() - ref).max() / np.abs(ref).max())
+
+
+def splits(M, N, K, dtype, gate_up=False):
+    return cabi.lib.cbk_gemm_partial_floats(CODE[dtype], M, N, K, int(gate_up)) > 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bits", [2, 3, 4])
+@pytest.mark.parametrize("M,N,K,gs", [(17, 100, 4096, 128), (32, 136, 4200, 96), (33, 256, 5128, 32),
+                                      (64, 128, 11008, 128), (65, 96, 2816, 64), (100, 300, 4328, 256),
+                                      (128, 260, 8192, 128), (257, 128, 6400, 512), (300, 1000, 3592, 128)])
+def test_split_gemm(hip, dtype, bits, M, N, K, gs):
+    assert splits(M, N, K, dtype)
+    w, W, b = make(N, K, bits, dtype, gs, 1, bias=True)
+    x = randx(M, K, dtype)
+    ref = E.act64(x.double().cpu().numpy() @ W.T + b, 1)
+    y = packed_linear(x, w, act="relu")
+    assert off(y, ref) < BAR[dtype]
+    for _ in range(3):                                     # the counters are back at zero, the order is fixed
+        assert torch.equal(packed_linear(x, w, act="relu"), y)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,gs", [(17, 100, 4096, 128), (40, 130, 4200, 64), (130, 64, 8200, 128)])
+def test_split_gate_up(hip, dtype, M, N, K, gs):
+    assert splits(M, N, K, dtype, True)
+    g, G, _ = make(N, K, 3, dtype, gs, 1)
+    u, U, _ = make(N, K, 3, dtype, gs, 2)
+    x = randx(M, K, dtype)
+    xd = x.double().cpu().numpy()
+    ref = E.round_to(E.silu64(xd @ G.T), dtype) * E.round_to(xd @ U.T, dtype)
+    # three roundings: each factor's, relative, and the product's
+    assert off(fused_gate_up(x, g, u), ref) < 3 * BAR[dtype]
+
+
+@pytest.mark.parametrize("M,N,K", [(20, 200, 4096), (50, 128, 5000), (129, 128, 4096)])
+def test_split_gemm_fractional_zeros(hip, M, N, K):
+    w, W, _ = make(N, K, 4, torch.float16, 128, 1, fractional=True)
+    x = randx(M, K, torch.float16)
+    assert off(packed_linear(x, w), x.double().cpu().numpy() @ W.T) < BAR[torch.float16]
+
+
+def test_unsplit_without_a_buffer(hip):
+    """cbk_packed_gemm has no partial buffer: the same call runs unsplit, the sums in another order."""
+    M, N, K = 48, 256, 4096
+    w, W, _ = make(N, K, 4, torch.float16, 128, 1)
+    x = randx(M, K, torch.float16)
+    out = torch.empty(M, N, dtype=torch.float16, device="cuda")
+    rc = cabi.lib.cbk_packed_gemm(x.data_ptr(), 0, M, K, w.packed.data_ptr(), w.scales.data_ptr(),
+                                  w.zeros.data_ptr(), None, N, 4, 128, 0, 1, out.data_ptr(), 0,
+                                  torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, cabi.last_error()
+    torch.cuda.synchronize()
+    assert off(out, x.double().cpu().numpy() @ W.T) < BAR[torch.float16]
+
+
+def test_split_gemm_streams_and_replays(hip):
+    """A split call on another stream, and captured: every replay, between eager calls, gives one
+    and the same result.  (A process that has used every counter window runs a new stream's or
+    capture's call unsplit, its sums in another order: the bar, not the bits, holds against eager.)"""
+    w, W, _ = make(512, 4096, 3, torch.float16, 128, 1)
+    x = randx(40, 4096, torch.float16)
+    ref = x.double().cpu().numpy() @ W.T
+    y = packed_linear(x, w)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        ys = packed_linear(x, w)
+    s.synchronize()
+    assert off(ys, ref) < BAR[torch.float16]
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        yg = packed_linear(x, w)
+    first = None
+    for _ in range(4):
+        yg.zero_()
+        g.replay()
+        assert torch.equal(packed_linear(x, w), y)
+        torch.cuda.synchronize()
+        first = yg.clone() if first is None else first
+        assert torch.equal(yg, first)
+    assert off(first, ref) < BAR[torch.float16]
