@@ -194,7 +194,9 @@ __device__ __forceinline__ void loads_setup(const GemmArgs& A, int m0, int n0, i
     const bool up_sz = GU && (wave & 3) >= 2;
     L.szr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<void*>(SZ_Q * wave >= 4 ? (up_sz ? A.z2 : A.z) : (up_sz ? A.s2 : A.s)), (short)0,
-        A.N * A.G * 2, 0x00020000);
+        // whole words: the range check drops a word that is not wholly inside, and with an odd
+        // N G the last column's last value is half of one (the word is the tensor's own)
+        (int)(((uint32_t)A.N * A.G * 2 + 3) & ~3u), 0x00020000);
 #pragma unroll
     for (int t = 0; t < G::W_Q; ++t) {
         const bool up_w = GU && WAVES * t + wave >= G::PPR;
@@ -517,7 +519,9 @@ __device__ __forceinline__ void read_w(const GemmArgs& A, const lds_t* lds, int 
         const uint32_t w = fdiv((uint32_t)(j * 256), A.divG) >> 3;       // j / (gs / 32)
         const lds_t* sb = lds + Lay<BITS, MB>::SZ_OFF + (w & 1) * SZ_BUF;
         const long span = (ci.cg + SZG * (long)w) & ~7L;
-        const int gi = (int)fdiv((uint32_t)((4 * s + ci.cix) * 32), A.divG);
+        // a chunk past K takes the last group's: what follows the tensor need not be finite, and
+        // not a number times the chunk's zero activations is none
+        const int gi = min((int)fdiv((uint32_t)((4 * s + ci.cix) * 32), A.divG), A.G - 1);
         l16* q = reinterpret_cast<l16*>(sb + ci.soff) + (int)(ci.cg + gi - span);
         r.s = q[0];
         r.z = q[BN * 16];

@@ -51,7 +51,8 @@ def splits(M, N, K, dtype, gate_up=False):
 @pytest.mark.parametrize("bits", [2, 3, 4])
 @pytest.mark.parametrize("M,N,K,gs", [(17, 100, 4096, 128), (32, 136, 4200, 96), (33, 256, 5128, 32),
                                       (64, 128, 11008, 128), (65, 96, 2816, 64), (100, 300, 4328, 256),
-                                      (128, 260, 8192, 128), (257, 128, 6400, 512), (300, 1000, 3592, 128)])
+                                      (128, 260, 8192, 128), (257, 128, 6400, 512), (300, 1000, 3592, 128),
+                                      (33, 257, 5128, 32), (20, 129, 4136, 64)])
 def test_split_gemm(hip, dtype, bits, M, N, K, gs):
     assert splits(M, N, K, dtype)
     w, W, b = make(N, K, bits, dtype, gs, 1, bias=True)
