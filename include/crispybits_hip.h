@@ -143,6 +143,17 @@ int cbk_fused_qkv_mixed(const void* x, int dtype, int64_t M, int64_t K,
                         int32_t* workspace, float* partial, void* out_q, void* out_k, void* out_v,
                         int device, void* stream);
 
+/* cbk_fused_qkv_mixed with the RoPE tables in fp32 (rope_f32) or in x's dtype, as a model hands
+ * them over, so that no conversion runs ahead of the call (additive). */
+int cbk_fused_qkv_rope(const void* x, int dtype, int64_t M, int64_t K,
+                       const int32_t* wq, const void* sq, const void* zq, const void* bq, int64_t nq,
+                       const int32_t* wk, const void* sk, const void* zk, const void* bk, int64_t nk,
+                       const int32_t* wv, const void* sv, const void* zv, const void* bv, int64_t nv,
+                       const void* rope_cos, const void* rope_sin, int rope_f32, int head_dim, int perm_hd,
+                       int bits_q, int bits_k, int bits_v, int group_size, int split_k, int rho,
+                       int32_t* workspace, float* partial, void* out_q, void* out_k, void* out_v,
+                       int device, void* stream);
+
 /* Prefill: out[M,N] = act(x . W-hat^T + bias).  With use_matrix_cores and fp16/bf16 x,
  * W-hat = RN_T((q - z) * s) runs on the 16-bit matrix cores; otherwise (fp32 x, or
  * use_matrix_cores = 0) W-hat is kept unrounded in fp32 and the products run on the fp32

@@ -369,16 +369,13 @@ def fused_qkv(x: torch.Tensor, q: PackedLinearWeight, k: PackedLinearWeight, v: 
         if perm != head_dim:
             raise ValueError("fused RoPE needs Q/K permuted with permute_for_rope(w, head_dim) "
                              "(install_bitmap(fuse_rope=True) does this)")
-        pre = x.shape[:-1]                    # one cos/sin row per activation row
-        cos2 = cos.expand(*pre, head_dim).reshape(M, head_dim)
-        sin2 = sin.expand(*pre, head_dim).reshape(M, head_dim)
+        cos2, sin2 = (t if t.shape == (M, head_dim) and lead is None    # one cos/sin row per activation row
+                      else t.expand(*x.shape[:-1], head_dim).reshape(M, head_dim) for t in (cos, sin))
     if M <= decode_threshold:
         pk = _k_splits(split_k, rho, M, q.out_features + k.out_features + v.out_features, q.in_features, x2)
-        rc = None if cos2 is None else cos2.float().contiguous()
-        rs = None if sin2 is None else sin2.float().contiguous()
         bits = q.bits if q.bits == k.bits == v.bits else (q.bits, k.bits, v.bits)
         outs = _C.fused_qkv(x2, q.packed, q.scales, q.zeros, q.bias, k.packed, k.scales, k.zeros, k.bias,
-                            v.packed, v.scales, v.zeros, v.bias, rc, rs, head_dim, perm, bits, q.in_features,
+                            v.packed, v.scales, v.zeros, v.bias, cos2, sin2, head_dim, perm, bits, q.in_features,
                             q.group_size, pk, rho, workspace)
     else:
         outs = _prefill_qkv(x2, q, k, v, cos2, sin2)

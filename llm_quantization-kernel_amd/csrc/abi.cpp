@@ -661,7 +661,7 @@ GemvArgs base_args(const void* x, int64_t M, int64_t K, int gs) {
 int qkv_common(const void* x, int dtype, int64_t M, int64_t K, const int32_t* wq, const void* sq, const void* zq,
                const void* bq, int64_t nq, const int32_t* wk, const void* sk, const void* zk, const void* bk,
                int64_t nk, const int32_t* wv, const void* sv, const void* zv, const void* bv, int64_t nv,
-               const float* rope_cos, const float* rope_sin, int head_dim, int perm_hd, int bits_q, int bits_k,
+               const void* rope_cos, const void* rope_sin, int rope_f32, int head_dim, int perm_hd, int bits_q, int bits_k,
                int bits_v, int group_size, int split_k, int rho, float* partial, void* out_q, void* out_k,
                void* out_v, int device, void* stream) {
     int rc = check_x(x, dtype, M, K);
@@ -695,6 +695,7 @@ int qkv_common(const void* x, int dtype, int64_t M, int64_t K, const int32_t* wq
     if (rope) {
         A.rope_cos = rope_cos;
         A.rope_sin = rope_sin;
+        A.rope_f32 = rope_f32;
         A.head_dim = head_dim;
     }
     const bool mixed = !(bits_q == bits_k && bits_k == bits_v);
@@ -900,7 +901,7 @@ int cbk_fused_qkv(const void* x, int dtype, int64_t M, int64_t K, const int32_t*
                   int split_k, int rho, int32_t* workspace, float* partial, void* out_q, void* out_k, void* out_v,
                   int device, void* stream) {
     (void)workspace;
-    return qkv_common(x, dtype, M, K, wq, sq, zq, bq, nq, wk, sk, zk, bk, nk, wv, sv, zv, bv, nv, rope_cos, rope_sin,
+    return qkv_common(x, dtype, M, K, wq, sq, zq, bq, nq, wk, sk, zk, bk, nk, wv, sv, zv, bv, nv, rope_cos, rope_sin, 1,
                       head_dim, perm_hd, bits, bits, bits, group_size, split_k, rho, partial, out_q, out_k, out_v,
                       device, stream);
 }
@@ -912,9 +913,21 @@ int cbk_fused_qkv_mixed(const void* x, int dtype, int64_t M, int64_t K, const in
                         int bits_q, int bits_k, int bits_v, int group_size, int split_k, int rho, int32_t* workspace,
                         float* partial, void* out_q, void* out_k, void* out_v, int device, void* stream) {
     (void)workspace;
-    return qkv_common(x, dtype, M, K, wq, sq, zq, bq, nq, wk, sk, zk, bk, nk, wv, sv, zv, bv, nv, rope_cos, rope_sin,
+    return qkv_common(x, dtype, M, K, wq, sq, zq, bq, nq, wk, sk, zk, bk, nk, wv, sv, zv, bv, nv, rope_cos, rope_sin, 1,
                       head_dim, perm_hd, bits_q, bits_k, bits_v, group_size, split_k, rho, partial, out_q, out_k,
                       out_v, device, stream);
+}
+
+int cbk_fused_qkv_rope(const void* x, int dtype, int64_t M, int64_t K, const int32_t* wq, const void* sq,
+                       const void* zq, const void* bq, int64_t nq, const int32_t* wk, const void* sk, const void* zk,
+                       const void* bk, int64_t nk, const int32_t* wv, const void* sv, const void* zv, const void* bv,
+                       int64_t nv, const void* rope_cos, const void* rope_sin, int rope_f32, int head_dim, int perm_hd,
+                       int bits_q, int bits_k, int bits_v, int group_size, int split_k, int rho, int32_t* workspace,
+                       float* partial, void* out_q, void* out_k, void* out_v, int device, void* stream) {
+    (void)workspace;
+    return qkv_common(x, dtype, M, K, wq, sq, zq, bq, nq, wk, sk, zk, bk, nk, wv, sv, zv, bv, nv, rope_cos, rope_sin,
+                      rope_f32, head_dim, perm_hd, bits_q, bits_k, bits_v, group_size, split_k, rho, partial, out_q,
+                      out_k, out_v, device, stream);
 }
 
 int cbk_packed_gemm(const void* x, int dtype, int64_t M, int64_t K, const int32_t* packed, const void* scales,

@@ -134,13 +134,13 @@ struct GemvArgs {
     int ntiles;            // fp32 matrix-core kernel: 16-row tiles
     FastDiv divP, divRW, divGS, divG, divT;   // by P, st_rw, gs / 32, gs / 128, ntiles
     Dst dst[3];
-    const float* rope_cos; // [M, head_dim] or nullptr
-    const float* rope_sin;
+    const void* rope_cos;  // [M, head_dim] or nullptr, fp32 or x's dtype (rope_f32)
+    const void* rope_sin;
     int head_dim, perm_hd;
     FastDiv divHD;         // by perm_hd (1 when the Q/K rows are not pair-interleaved)
     int mtiles, jobs;      // fp32 matrix-core kernel: 16-row batch tiles, jobs
     int bits[3];           // code width of each projection
-    int pad_;
+    int rope_f32;          // the RoPE tables are fp32
 };
 
 // ---------------------------------------------------------------- projection views
@@ -244,9 +244,16 @@ __device__ __forceinline__ void qkv_finish(const GemvArgs& A, int b, int v0, flo
         const int d = (r - head * hd) >> 1;               // < hd / 2
         const long o = (long)b * D.ld + head * hd + d;    // original rows o and o + hd / 2
         if (A.rope_cos != nullptr) {                      // head_dim == perm_hd (host check)
-            const float* cs = A.rope_cos + (long)b * hd;
-            const float* sn = A.rope_sin + (long)b * hd;
-            const float c0 = cs[d], s0 = sn[d], c1 = cs[d + half], s1 = sn[d + half];
+            const long i0 = (long)b * hd + d, i1 = i0 + half;
+            float c0, s0, c1, s1;
+            if (A.rope_f32) {
+                const float* cs = reinterpret_cast<const float*>(A.rope_cos);
+                const float* sn = reinterpret_cast<const float*>(A.rope_sin);
+                c0 = cs[i0], s0 = sn[i0], c1 = cs[i1], s1 = sn[i1];
+            } else {
+                c0 = load_f<DT>(A.rope_cos, i0), s0 = load_f<DT>(A.rope_sin, i0);
+                c1 = load_f<DT>(A.rope_cos, i1), s1 = load_f<DT>(A.rope_sin, i1);
+            }
             store_f<DT>(D.y, o, y0 * c0 - y1 * s0);
             store_f<DT>(D.y, o + half, y1 * c1 + y0 * s1);
         } else {

@@ -260,8 +260,12 @@ std::vector<Tensor> fused_qkv(const Tensor& x, const Tensor& wq, const Tensor& s
                     "(ops.permute_for_rope / install_bitmap(fuse_rope=True))");
         TORCH_CHECK(rope_sin.has_value() && rope_cos->sizes() == rope_sin->sizes(), "cos/sin shape mismatch");
         TORCH_CHECK(rope_cos->numel() == B * head_dim, "cos/sin must be [B, head_dim] (one row per x row)");
-        rc = rope_cos->to(x.device(), at::kFloat).contiguous();
-        rs = rope_sin->to(x.device(), at::kFloat).contiguous();
+        // tables in fp32 or in x's dtype are read as they are
+        const bool as_is = rope_cos->scalar_type() == rope_sin->scalar_type() &&
+                           rope_cos->scalar_type() == x.scalar_type() && rope_cos->device() == x.device() &&
+                           rope_sin->device() == x.device();
+        rc = (as_is ? *rope_cos : rope_cos->to(x.device(), at::kFloat)).contiguous();
+        rs = (as_is ? *rope_sin : rope_sin->to(x.device(), at::kFloat)).contiguous();
     }
     const int64_t nq = wq.size(0), nk = wk.size(0), nv = wv.size(0);
     const void* pq = bias_ptr(bq, x, nq);
@@ -270,29 +274,18 @@ std::vector<Tensor> fused_qkv(const Tensor& x, const Tensor& wq, const Tensor& s
     int32_t* ws = workspace_ptr(workspace, x);
     // one allocation carved into three contiguous [B, n] outputs (each its own block of it)
     const Tensor flat = at::empty({B * (nq + nk + nv)}, x.options());
-    std::vector<Tensor> outs = {flat.narrow(0, 0, B * nq).view({B, nq}), flat.narrow(0, B * nq, B * nk).view({B, nk}),
-                                flat.narrow(0, B * (nq + nk), B * nv).view({B, nv})};
+    std::vector<Tensor> outs = {flat.as_strided({B, nq}, {nq, 1}, 0), flat.as_strided({B, nk}, {nk, 1}, B * nq),
+                                flat.as_strided({B, nv}, {nv, 1}, B * (nq + nk))};
     if (B == 0) return outs;
     const Tensor part = partial_for(x, B, nq + nk + nv, in_features, group_size, split_k);
     const int dev = x.get_device();
-    const float* c = rope ? rc.data_ptr<float>() : nullptr;
-    const float* s = rope ? rs.data_ptr<float>() : nullptr;
-    const int hd = rope ? (int)head_dim : 0;
-    float* p = static_cast<float*>(tensor_ptr(part));
-    if (b3[0] == b3[1] && b3[1] == b3[2]) {
-        ok(cbk_fused_qkv(x.data_ptr(), dtype_of(x.scalar_type()), B, in_features, wq.data_ptr<int32_t>(),
-                         sq.data_ptr(), zq.data_ptr(), pq, nq, wk.data_ptr<int32_t>(), sk.data_ptr(), zk.data_ptr(),
-                         pk, nk, wv.data_ptr<int32_t>(), sv.data_ptr(), zv.data_ptr(), pv, nv, c, s, hd,
-                         (int)perm_hd, (int)b3[0], (int)group_size, (int)split_k, (int)rho, ws, p,
-                         outs[0].data_ptr(), outs[1].data_ptr(), outs[2].data_ptr(), dev, stream_of(dev)));
-    } else {
-        ok(cbk_fused_qkv_mixed(x.data_ptr(), dtype_of(x.scalar_type()), B, in_features, wq.data_ptr<int32_t>(),
-                               sq.data_ptr(), zq.data_ptr(), pq, nq, wk.data_ptr<int32_t>(), sk.data_ptr(),
-                               zk.data_ptr(), pk, nk, wv.data_ptr<int32_t>(), sv.data_ptr(), zv.data_ptr(), pv, nv,
-                               c, s, hd, (int)perm_hd, (int)b3[0], (int)b3[1], (int)b3[2], (int)group_size,
-                               (int)split_k, (int)rho, ws, p, outs[0].data_ptr(), outs[1].data_ptr(),
-                               outs[2].data_ptr(), dev, stream_of(dev)));
-    }
+    ok(cbk_fused_qkv_rope(x.data_ptr(), dtype_of(x.scalar_type()), B, in_features, wq.data_ptr<int32_t>(),
+                          sq.data_ptr(), zq.data_ptr(), pq, nq, wk.data_ptr<int32_t>(), sk.data_ptr(), zk.data_ptr(),
+                          pk, nk, wv.data_ptr<int32_t>(), sv.data_ptr(), zv.data_ptr(), pv, nv, tensor_ptr(rc),
+                          tensor_ptr(rs), rope && rc.scalar_type() == at::kFloat ? 1 : 0, rope ? (int)head_dim : 0,
+                          (int)perm_hd, (int)b3[0], (int)b3[1], (int)b3[2], (int)group_size, (int)split_k, (int)rho,
+                          ws, static_cast<float*>(tensor_ptr(part)), outs[0].data_ptr(), outs[1].data_ptr(),
+                          outs[2].data_ptr(), dev, stream_of(dev)));
     return outs;
 }
 

@@ -27,6 +27,9 @@ SIGS = {
     "cbk_fused_qkv_mixed": (_I, [_P, _I, _L, _L,
                                  _P, _P, _P, _P, _L, _P, _P, _P, _P, _L, _P, _P, _P, _P, _L,
                                  _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _P]),
+    "cbk_fused_qkv_rope": (_I, [_P, _I, _L, _L,
+                                _P, _P, _P, _P, _L, _P, _P, _P, _P, _L, _P, _P, _P, _P, _L,
+                                _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _P]),
     "cbk_packed_gemm": (_I, [_P, _I, _L, _L, _P, _P, _P, _P, _L, _I, _I, _I, _I, _P, _I, _P]),
     "cbk_gemm_qkv_partial_floats": (_L, [_I, _L, _L, _L, _L, _L]),
     "cbk_packed_gemm_qkv": (_I, [_P, _I, _L, _L,

@@ -90,3 +90,22 @@ def test_qkv_gemm_large_batch(hip):
     one, three = check(x, q, k, v, (cos.expand(2, -1, -1), sin.expand(2, -1, -1), 128))
     assert one[0].shape == (2, 1030, 1024)
     assert torch.equal(one[2], three[2])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,K,gs", [(1, 512, 128), (2, 512, 64), (3, 1024, 128), (16, 512, 128), (5, 500, 32)])
+def test_decode_tables_in_x_dtype(hip, dtype, M, K, gs):
+    """RoPE tables in x's dtype are read as they are: the bits of the same tables in fp32, on each
+    decode kernel and with a K split."""
+    hd = 32
+    q, k, v = (weight(64, K, 3, dtype, gs, i) for i in range(3))
+    q, k = permute_for_rope(q, hd), permute_for_rope(k, hd)
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(3)).to(dtype).cuda()
+    cos, sin = tables(M, hd, dtype)
+    for split_k in (None, 2):
+        a = fused_qkv(x, q, k, v, split_k, rope=(cos, sin, hd))
+        b = fused_qkv(x, q, k, v, split_k, rope=(cos.float(), sin.float(), hd))
+        assert all(torch.equal(s, t) for s, t in zip(a, b))
+    cols = torch.cat([cos, sin], dim=1)                    # tables that are views of one tensor
+    a = fused_qkv(x, q, k, v, rope=(cols[:, :hd], cols[:, hd:], hd))
+    assert all(torch.equal(s, t) for s, t in zip(a, fused_qkv(x, q, k, v, rope=(cos, sin, hd))))
