@@ -23,7 +23,7 @@ LIB_NAME = "libcrispybits_hip.so"
 LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
 ARCH = os.environ.get("CRISPYBITS_ARCH", "gfx950")
 
-SOURCES = ["abi.cpp", "gemv_stream.hip", "gemv_any.hip", "gemm.hip", "gemm_f16.cpp", "gemm_f16_mb1.hip",
+SOURCES = ["abi.cpp", "gemv_stream.hip", "gemv_bsub.hip", "gemv_any.hip", "gemm.hip", "gemm_f16.cpp", "gemm_f16_mb1.hip",
            "gemm_f16_mb2.hip", "gemm_f16_mb4.hip", "gemm_f16_mb4s.hip", "gemm_f32.hip",
            "unpack.hip", "quant.hip", "probe.hip"]
 

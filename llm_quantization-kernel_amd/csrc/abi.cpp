@@ -325,16 +325,20 @@ StreamPlan plan_stream(const GemvArgs& A, int dtype, int mode, bool mixed, int s
 struct BStreamPlan {
     bool ok = false;
     bool filled = false;         // chosen by bstream_fill
-    int P = 1, ks = 1, rw = 1, bsu = 4, grid = 0, lds = 0;
+    int P = 1, ks = 1, rw = 1, bsu = 4, grid = 0, lds = 0, sub = 1;
 };
 
 // LDS of a batched streaming workgroup: the staged activations (xr operand rows per batch
 // row: 2 for fp32, hi and lo), two per-unit sums (three for bf16 and fp32: the per-unit
 // prescale) for 16 operand rows, and the row totals.
-int64_t bstream_lds(int64_t ks, int64_t M, int64_t rw, int bsu, bool bf, int xr = 1) {
+// sub: sub-units a unit (bstream_sub), each with its two sums.
+int64_t bstream_lds(int64_t ks, int64_t M, int64_t rw, int bsu, bool bf, int xr, int sub) {
     const int64_t nu = ks * bsu;
-    return 64 * 4 * nu * M * xr + (bf ? 3 : 2) * 16 * nu * 4 + 4 * ks * M * 16 * rw;
+    return 64 * 4 * nu * M * xr + (2 * sub + (bf ? 1 : 0)) * 16 * nu * 4 + 4 * ks * M * 16 * rw;
 }
+
+// Sub-units of a 128-code unit that lie in one group each.
+int bstream_sub(int gs) { return gs % 128 == 0 ? 1 : (gs % 64 == 0 ? 2 : 4); }
 
 // Row groups: enough threads to stage the activations two items per thread (4 bsu M
 // items over 64 threads per wave), and for gate-up an even count (one wave per
@@ -350,12 +354,12 @@ int bstream_rw(int64_t M, int bsu, bool gateup) {
 int bstream_max_waves(int bsu, bool bf) { return bf && bsu == 8 ? 12 : 16; }
 
 // K splits of the batched streaming kernel for slices of bsu units.
-int bstream_splits(int64_t C, int64_t M, int split_k, int rw, int bsu, bool bf, int xr = 1) {
+int bstream_splits(int64_t C, int64_t M, int split_k, int rw, int bsu, bool bf, int xr, int sub) {
     const int64_t U = ceil_div(C, 4);
     int64_t P = std::max<int64_t>(1, std::min<int64_t>(split_k, U));
     while (P < U) {
         const int64_t ks = ceil_div(ceil_div(U, P), bsu);
-        if (ks * rw <= bstream_max_waves(bsu, bf) && bstream_lds(ks, M, rw, bsu, bf, xr) <= LDS_BUDGET) break;
+        if (ks * rw <= bstream_max_waves(bsu, bf) && bstream_lds(ks, M, rw, bsu, bf, xr, sub) <= LDS_BUDGET) break;
         ++P;
     }
     return (int)P;
@@ -366,7 +370,8 @@ int bstream_splits(int64_t C, int64_t M, int split_k, int rw, int bsu, bool bf, 
 // by at most two threads, an even number of row groups for gate-up, the LDS, one
 // projection per workgroup for mixed widths, 32-bit indices, and with P > 1 a counter
 // per row block in one window (the splits combine in the dispatch).
-BStreamPlan bstream_make(const GemvArgs& A, int mode, bool mixed, int P, int bsu, int rw, bool bf, int xr = 1) {
+BStreamPlan bstream_make(const GemvArgs& A, int mode, bool mixed, int P, int bsu, int rw, bool bf, int xr,
+                         int sub) {
     BStreamPlan bp;
     const int64_t U = ceil_div(A.C, 4);
     if (P < 1 || P > U || (int64_t)U * P >= (1ll << 32)) return bp;
@@ -376,7 +381,8 @@ BStreamPlan bstream_make(const GemvArgs& A, int mode, bool mixed, int P, int bsu
     bp.rw = rw;
     bp.ks = (int)ceil_div(ceil_div(U, P), bsu);
     if (bp.ks * rw > bstream_max_waves(bsu, bf)) return bp;
-    bp.lds = (int)bstream_lds(bp.ks, A.M, rw, bsu, bf, xr);
+    bp.sub = sub;
+    bp.lds = (int)bstream_lds(bp.ks, A.M, rw, bsu, bf, xr, sub);
     if (bp.lds > LDS_BUDGET) return bp;
     const int rb = 16 * rw;
     if (mixed && (A.src[0].n % rb != 0 || A.src[1].n % rb != 0)) return bp;
@@ -399,13 +405,13 @@ BStreamPlan bstream_make(const GemvArgs& A, int mode, bool mixed, int P, int bsu
 constexpr int BSTREAM_CU_TARGET = 256;
 constexpr int BSTREAM_FILL_SPLITS = 4;
 
-BStreamPlan bstream_fill(const GemvArgs& A, int mode, bool mixed, int P0, bool bf, int xr = 1) {
+BStreamPlan bstream_fill(const GemvArgs& A, int mode, bool mixed, int P0, bool bf, int xr, int sub) {
     BStreamPlan best;
     int64_t best_key = INT64_MAX;
     for (int P = P0; P < P0 + BSTREAM_FILL_SPLITS; ++P) {
-        for (int bsu : {4, 8}) {
+        for (int bsu = 4; bsu <= (sub == 1 ? 8 : 4); bsu += 4) {
             for (int rw = 1; rw <= 16; ++rw) {
-                const BStreamPlan c = bstream_make(A, mode, mixed, P, bsu, rw, bf, xr);
+                const BStreamPlan c = bstream_make(A, mode, mixed, P, bsu, rw, bf, xr, sub);
                 if (!c.ok) continue;
                 const int64_t dist = std::abs((int64_t)c.grid - BSTREAM_CU_TARGET);
                 const int64_t key = ((dist * 64 + (P - P0)) * 2 + (bsu == 8)) * 32 + rw;
@@ -421,14 +427,14 @@ BStreamPlan bstream_fill(const GemvArgs& A, int mode, bool mixed, int P0, bool b
 
 // The unsplit-first plan before any widening for the CU count: 4-unit slices with the
 // fewest splits that fit, or 8-unit slices where those need fewer splits.
-BStreamPlan bstream_base(int64_t M, int64_t C, int split_k, bool gateup, bool bf, int xr = 1) {
+BStreamPlan bstream_base(int64_t M, int64_t C, int split_k, bool gateup, bool bf, int xr, int sub) {
     BStreamPlan bp;
     bp.bsu = 4;
     bp.rw = bstream_rw(M, 4, gateup);
-    bp.P = bstream_splits(C, M, split_k, bp.rw, 4, bf, xr);
-    if (bp.P > std::max(split_k, 1)) {           // 4-unit slices would add a split: try 8
+    bp.P = bstream_splits(C, M, split_k, bp.rw, 4, bf, xr, sub);
+    if (bp.P > std::max(split_k, 1) && sub == 1) {   // 4-unit slices would add a split: try 8
         const int rw8 = bstream_rw(M, 8, gateup);
-        const int p8 = bstream_splits(C, M, split_k, rw8, 8, bf, xr);
+        const int p8 = bstream_splits(C, M, split_k, rw8, 8, bf, xr, sub);
         if (p8 < bp.P) {
             bp.bsu = 8;
             bp.rw = rw8;
@@ -455,7 +461,7 @@ BStreamPlan plan_bstream(const GemvArgs& A, int dtype, int mode, bool mixed, int
     const bool bf = dtype != CBK_F16;
     const int xr = dtype == CBK_F32 ? 2 : 1, xe = dtype == CBK_F32 ? 4 : 2;
     const int mmin = dtype == CBK_F32 ? 2 : 3;         // below: the batch-1/2 streaming kernel
-    bool ok = A.M >= mmin && A.M * xr <= 16 && valid_dtype(dtype) && A.gs % 128 == 0 && A.K % 8 == 0 &&
+    bool ok = A.M >= mmin && A.M * xr <= 16 && valid_dtype(dtype) && A.gs % 32 == 0 && A.K % 8 == 0 &&
               reinterpret_cast<uintptr_t>(A.x) % 16 == 0 && (int64_t)A.M * A.K * xe < lim;
     for (int i = 0; i < 3; ++i)
         ok = ok && (int64_t)A.src[i].n * A.src[i].wpr * 4 < lim && (int64_t)A.src[i].n * A.G * xe < lim;
@@ -463,9 +469,10 @@ BStreamPlan plan_bstream(const GemvArgs& A, int dtype, int mode, bool mixed, int
     if (!ok) return bp;
     const bool gateup = mode == CBK_MODE_GATEUP;
     const int64_t U = ceil_div(A.C, 4);
-    bp = bstream_base(A.M, A.C, split_k, gateup, bf, xr);
+    const int sub = bstream_sub(A.gs);
+    bp = bstream_base(A.M, A.C, split_k, gateup, bf, xr, sub);
     if (bstream_fills(bp, A.V)) {
-        BStreamPlan fill = bstream_fill(A, mode, mixed, std::max(split_k, 1), bf, xr);
+        BStreamPlan fill = bstream_fill(A, mode, mixed, std::max(split_k, 1), bf, xr, sub);
         if (fill.ok) {
             fill.filled = true;
             return fill;
@@ -476,24 +483,24 @@ BStreamPlan plan_bstream(const GemvArgs& A, int dtype, int mode, bool mixed, int
     // blocks would give each CU 2.5 or more workgroups take 8-unit slices and the
     // fewest workgroups that still cover the CUs (W3 4096 -> 11008: batch 8 13.2 -> 11.1
     // us, batch 16 18.8 -> 14.5), and gate-up takes 8-unit slices (batch 4 20.4 -> 15.6).
-    if (bp.P == 1 && cus > 0) {
+    if (bp.P == 1 && cus > 0 && sub == 1) {
         const int64_t U8 = ceil_div(U, 8);
         const int mw = bstream_max_waves(8, bf);
         if (mode == CBK_MODE_GEMV && !mixed && ceil_div(A.V, 16) >= (5 * (int64_t)cus) / 2) {
             int rw = (int)std::max<int64_t>(bstream_rw(A.M, 8, false), ceil_div(ceil_div(A.V, 16), cus));
-            if (U8 * rw <= mw && bstream_lds(U8, A.M, rw, 8, bf, xr) <= LDS_BUDGET) {
+            if (U8 * rw <= mw && bstream_lds(U8, A.M, rw, 8, bf, xr, sub) <= LDS_BUDGET) {
                 bp.bsu = 8;
                 bp.rw = rw;
             }
         } else if (gateup) {
             const int rw = bstream_rw(A.M, 8, true);
-            if (U8 * rw <= mw && bstream_lds(U8, A.M, rw, 8, bf, xr) <= LDS_BUDGET) {
+            if (U8 * rw <= mw && bstream_lds(U8, A.M, rw, 8, bf, xr, sub) <= LDS_BUDGET) {
                 bp.bsu = 8;
                 bp.rw = rw;
             }
         }
     }
-    return bstream_make(A, mode, mixed, bp.P, bp.bsu, bp.rw, bf, xr);
+    return bstream_make(A, mode, mixed, bp.P, bp.bsu, bp.rw, bf, xr, sub);
 }
 
 // Kernels (per device) whose dynamic-LDS limit has been raised to the whole budget.  The
@@ -524,7 +531,10 @@ struct DecodeLaunch {
     int grid = 0, block = 0, lds = 0, P = 1;
 };
 
-DecodeLaunch plan_decode(GemvArgs& A, int dtype, int mode, bool mixed, int split_k, int rho, int cus) {
+// fine: groups finer than a 128-code unit may take the batched streaming kernel, whose splits need
+// a partial buffer where the fp32 matrix-core kernel needs none.
+DecodeLaunch plan_decode(GemvArgs& A, int dtype, int mode, bool mixed, int split_k, int rho, int cus,
+                         bool fine = true) {
     (void)rho;
     DecodeLaunch L;
     // batch 1 and 2: the streaming kernel
@@ -546,16 +556,19 @@ DecodeLaunch plan_decode(GemvArgs& A, int dtype, int mode, bool mixed, int split
     }
     // batch 3..16: the K-split streaming kernel (unsplit, or splits that combine in the
     // dispatch)
-    const BStreamPlan bp = plan_bstream(A, dtype, mode, mixed, split_k, cus);
+    const BStreamPlan bp =
+        fine || bstream_sub(A.gs) == 1 ? plan_bstream(A, dtype, mode, mixed, split_k, cus) : BStreamPlan();
     if (bp.ok) {
         A.P = bp.P;
         A.st_ks = bp.ks;
         A.st_rw = bp.rw;
         A.divP = make_fastdiv((uint32_t)A.P);
         A.divRW = make_fastdiv((uint32_t)A.st_rw);
-        A.divG = make_fastdiv((uint32_t)(A.gs / 128));
-        L.family = CBK_KERNEL_BSTREAM;
-        L.f = gemv_bstream_kernel_for(mode, A.bits[0], mixed, bp.bsu, dtype);
+        A.divG = make_fastdiv((uint32_t)(A.gs * bp.sub / 128));
+        // the builds for finer groups count as the generic family: the calls that the 128-code
+        // units do not take
+        L.family = bp.sub == 1 ? CBK_KERNEL_BSTREAM : CBK_KERNEL_GENERIC;
+        L.f = gemv_bstream_kernel_for(mode, A.bits[0], mixed, bp.bsu, dtype, bp.sub);
         L.grid = bp.grid;
         L.block = 64 * bp.ks * bp.rw;
         L.lds = bp.lds;
@@ -592,12 +605,14 @@ bool combines_in_dispatch(const DecodeLaunch& L) {
 
 // Common body of the three decode entry points.
 int run_decode(GemvArgs& A, int dtype, int mode, bool mixed, int split_k, int rho, float* partial, int device,
-               void* stream) {
+               void* stream, bool fine = true) {
     DeviceGuard guard(device);
     if (guard.err != hipSuccess) return hip_fail(guard.err, "set device");
     const int cus = cu_count(device);
     if (cus <= 0) return fail(CBK_EHIP, "cannot query the compute-unit count of device %d", device);
-    const DecodeLaunch L = plan_decode(A, dtype, mode, mixed, split_k, rho, cus);
+    DecodeLaunch L = plan_decode(A, dtype, mode, mixed, split_k, rho, cus, fine);
+    if (A.P > 1 && !partial && bstream_sub(A.gs) > 1)    // the plan of a caller without a buffer
+        L = plan_decode(A, dtype, mode, mixed, split_k, rho, cus, false);
     if (L.family == CBK_KERNEL_GENERIC && (int64_t)A.ntiles * A.mtiles * A.P >= (1ll << 31))
         return fail(CBK_EINVAL, "packed_gemv: problem too large for 32-bit job indexing");
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
@@ -772,20 +787,25 @@ int cbk_max_rho(int device, int bits, int mode, int* out) {
     return CBK_OK;
 }
 
-int64_t cbk_gemv_partial_floats(int dtype, int64_t M, int64_t V, int64_t K, int group_size, int split_k) {
+static int64_t partial_floats(int dtype, int64_t M, int64_t V, int64_t K, int group_size, int split_k, bool fine) {
     if (M <= 0 || V <= 0 || K <= 0 || group_size <= 0 || split_k < 1) return 0;
     int P = plan_any(M, V, K, split_k).P;
     if (M <= 2) P = std::max(P, stream_splits(ceil_div(K, 32), split_k, stream_max_slices((int)M, dtype)));
     const int xr = dtype == CBK_F32 ? 2 : 1;
-    if (M >= (dtype == CBK_F32 ? 2 : 3) && M * xr <= 16) {  // 4-unit slices split at least as often as 8-unit ones; gate-up rows
+    if (M >= (dtype == CBK_F32 ? 2 : 3) && M * xr <= 16 && (fine || bstream_sub(group_size) == 1)) {  // 4-unit slices split at least as often as 8-unit ones; gate-up rows
         const int64_t C = ceil_div(K, 32);
         const bool bf = dtype != CBK_F16;
-        P = std::max(P, bstream_splits(C, M, split_k, bstream_rw(M, 4, true), 4, bf, xr));
+        const int sub = bstream_sub(group_size);
+        P = std::max(P, bstream_splits(C, M, split_k, bstream_rw(M, 4, true), 4, bf, xr, sub));
         for (bool gateup : {false, true})     // bstream_fill takes at most P0 + 3 splits
-            if (bstream_fills(bstream_base(M, C, split_k, gateup, bf, xr), V))
+            if (bstream_fills(bstream_base(M, C, split_k, gateup, bf, xr, sub), V))
                 P = std::max<int64_t>(P, std::min<int64_t>(ceil_div(C, 4), split_k + BSTREAM_FILL_SPLITS - 1));
     }
     return P > 1 ? (int64_t)P * M * V : 0;
+}
+
+int64_t cbk_gemv_partial_floats(int dtype, int64_t M, int64_t V, int64_t K, int group_size, int split_k) {
+    return partial_floats(dtype, M, V, K, group_size, split_k, true);
 }
 
 int cbk_packed_gemv(const void* x, int dtype, int64_t M, int64_t K, const int32_t* packed, const void* scales,
@@ -851,7 +871,10 @@ int cbk_packed_gemv_noalloc(const void* x, int dtype, int64_t M, int64_t K, cons
     if (split_k < 1) return fail(CBK_EINVAL, "split_k must be >= 1");
     if (act < 0 || act > 2) return fail(CBK_EINVAL, "act must be 0 (none), 1 (relu) or 2 (silu)");
     if (!out) return fail(CBK_EINVAL, "packed_gemv_noalloc: out must be non-null");
-    const int64_t need = cbk_gemv_partial_floats(dtype, M, N, K, group_size, split_k);
+    // fine groups: a plan whose splits outgrow the scratch gives way to the one that needs fewer
+    int64_t need = partial_floats(dtype, M, N, K, group_size, split_k, true);
+    const bool fine = need <= NOALLOC_PARTIAL_FLOATS;
+    if (!fine) need = partial_floats(dtype, M, N, K, group_size, split_k, false);
     if (need > NOALLOC_PARTIAL_FLOATS)
         return fail(CBK_EINVAL,
                     "packed_gemv_noalloc: split-K partial sums need %lld floats, above the %lld-float device "
@@ -868,7 +891,8 @@ int cbk_packed_gemv_noalloc(const void* x, int dtype, int64_t M, int64_t K, cons
     repeat_proj0(A);
     A.V = (int)N;
     A.act = act;
-    return run_decode(A, dtype, CBK_MODE_GEMV, false, split_k, rho, need > 0 ? part : nullptr, device, stream);
+    return run_decode(A, dtype, CBK_MODE_GEMV, false, split_k, rho, need > 0 ? part : nullptr, device, stream,
+                      fine);
 }
 
 int cbk_fused_gate_up(const void* x, int dtype, int64_t M, int64_t K, const int32_t* wg, const void* sg,

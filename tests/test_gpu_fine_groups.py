@@ -1,0 +1,105 @@
+"""Batched decode with groups finer than 128 codes on the streaming kernel's sub-unit builds
+(multiples of 64, and of 32), against the oracle.
+
+The bars: one output rounding (2^-11 fp16, 2^-8 bf16) of the largest output plus 1e-4 for the fp32
+sums and the operands' staging; fp32 1e-6, four times the kernel's error against 64 bits."""
+import numpy as np
+import pytest
+import torch
+
+import cabi
+from crispybits_kernels import PackedLinearWeight, fused_gate_up, fused_qkv, packed_linear
+from crispybits_kernels.io import from_packed_dict
+from crispybits_kernels.reference import pack_linear_dict
+from oracle import emulator as E
+
+pytestmark = pytest.mark.gpu
+
+BAR = {torch.float16: 2.0 ** -11 + 1e-4, torch.bfloat16: 2.0 ** -8 + 1e-4, torch.float32: 1e-6}
+
+
+def make(N, K, bits, dtype, gs, seed=1, bias=False, fractional=False):
+    g = torch.Generator().manual_seed(seed)
+    b = torch.randn(N, generator=g) if bias else None
+    d = pack_linear_dict(torch.randn(N, K, generator=g) * 0.05, bits, gs, b, dtype)
+    if fractional:
+        d["zeros"] = d["zeros"] + 0.375
+    W = E.dequant64(d["packed"].numpy(), d["scales"].to(dtype).double().numpy(),
+                    d["zeros"].to(dtype).double().numpy(), bits, K, gs)
+    return from_packed_dict(d, "cuda", dtype), W, 0.0 if b is None else b.to(dtype).double().numpy()
+
+
+def randx(M, K, dtype, seed=3):
+    return torch.randn(M, K, generator=torch.Generator().manual_seed(seed)).to(dtype).cuda()
+
+
+def off(y, ref):
+    return float(np.abs(y.float().cpu().double().numpy() - ref).max() / np.abs(ref).max())
+
+
+@pytest.mark.parametrize("dtype,M", [(torch.float16, 3), (torch.float16, 16), (torch.bfloat16, 5),
+                                     (torch.bfloat16, 16), (torch.float32, 2), (torch.float32, 8)])
+@pytest.mark.parametrize("bits", [2, 3, 4])
+@pytest.mark.parametrize("N,K,gs", [(48, 2048, 64), (100, 1000, 64), (33, 4128, 32), (300, 640, 96), (17, 96, 32),
+                                    (64, 4104, 192), (40, 11008, 64), (80, 2080, 160)])
+def test_fine_groups(hip, dtype, M, bits, N, K, gs):
+    w, W, b = make(N, K, bits, dtype, gs, bias=True)
+    x = randx(M, K, dtype)
+    ref = E.act64(x.double().cpu().numpy() @ W.T + b, 2)
+    for split_k in (None, 3):
+        y = packed_linear(x, w, split_k, act="silu")
+        assert off(y, ref) < BAR[dtype]
+        assert torch.equal(packed_linear(x, w, split_k, act="silu"), y)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("gs", [32, 64])
+def test_fine_groups_fused(hip, dtype, gs):
+    M, K = 6, 1056
+    x = randx(M, K, dtype)
+    xd = x.double().cpu().numpy()
+    ws = [make(n, K, b, dtype, gs, i) for i, (n, b) in enumerate(((96, 4), (48, 2), (48, 3)))]
+    for o, (_, W, _) in zip(fused_qkv(x, *(w[0] for w in ws)), ws):
+        assert off(o, xd @ W.T) < BAR[dtype]
+    g, G, _ = make(100, K, 3, dtype, gs, 5, fractional=True)
+    u, U, _ = make(100, K, 3, dtype, gs, 6, fractional=True)
+    assert off(fused_gate_up(x, g, u), E.silu64(xd @ G.T) * (xd @ U.T)) < BAR[dtype]
+
+
+def test_fine_groups_at_the_scratch_limit(hip):
+    """A no-allocation call whose splits would outgrow the device scratch, and a call without a
+    partial buffer, take the plan that needs none: accepted, the same result within the bar."""
+    M, gs = 16, 64
+    n, k = 40, 32768                                       # a plan with splits, few rows
+    assert cabi.lib.cbk_gemv_partial_floats(0, M, n, k, gs, 1) > 0
+    w, W, _ = make(n, k, 2, torch.float16, gs)
+    x = randx(M, k, torch.float16)
+    out = torch.empty(M, n, dtype=torch.float16, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    ref = x.double().cpu().numpy() @ W.T
+    rc = cabi.lib.cbk_packed_gemv(x.data_ptr(), 0, M, k, w.packed.data_ptr(), w.scales.data_ptr(),
+                                  w.zeros.data_ptr(), None, n, 2, gs, 1, 1, 0, None, None, out.data_ptr(), 0, stream)
+    assert rc == 0, cabi.last_error()
+    torch.cuda.synchronize()
+    assert off(out, ref) < BAR[torch.float16]
+    out.zero_()
+    rc = cabi.lib.cbk_packed_gemv_noalloc(x.data_ptr(), 0, M, k, w.packed.data_ptr(), w.scales.data_ptr(),
+                                          w.zeros.data_ptr(), None, n, 2, gs, 1, 1, 0, out.data_ptr(), 0, stream)
+    assert rc == 0, cabi.last_error()
+    torch.cuda.synchronize()
+    assert off(out, ref) < BAR[torch.float16]
+    # past the scratch (P x 16 x 40000 floats): against the buffered call, random codes
+    n, k = 40000, 8192
+    assert cabi.lib.cbk_gemv_partial_floats(0, M, n, k, gs, 1) > 1 << 21
+    g = torch.Generator(device="cuda").manual_seed(1)
+    packed = torch.randint(-2 ** 31, 2 ** 31 - 1, (n, k // 16), generator=g, device="cuda", dtype=torch.int32)
+    scales = (torch.rand(n, k // gs, generator=g, device="cuda") + 0.5).half() / 64
+    zeros = torch.full_like(scales, 2.0)
+    x = randx(M, k, torch.float16)
+    y = packed_linear(x, PackedLinearWeight(packed, scales, zeros, 2, gs, k, n))
+    out = torch.empty(M, n, dtype=torch.float16, device="cuda")
+    rc = cabi.lib.cbk_packed_gemv_noalloc(x.data_ptr(), 0, M, k, packed.data_ptr(), scales.data_ptr(),
+                                          zeros.data_ptr(), None, n, 2, gs, 1, 1, 0, out.data_ptr(), 0, stream)
+    assert rc == 0, cabi.last_error()
+    torch.cuda.synchronize()
+    assert off(out, y.double().cpu().numpy()) < 2 * BAR[torch.float16]      # two results, a rounding each
