@@ -403,6 +403,7 @@ BStreamPlan bstream_make(const GemvArgs& A, int mode, bool mixed, int P, int bsu
 // groups); 4096^2 batch 16 10.1 -> 8.9 (P = 2).  The target is a constant -- the CU count
 // of every gfx950 part -- so cbk_gemv_partial_floats can bound P without a device.
 constexpr int BSTREAM_CU_TARGET = 256;
+constexpr int64_t BSTREAM_FINE_CODES = 1 << 21;
 constexpr int BSTREAM_FILL_SPLITS = 4;
 
 BStreamPlan bstream_fill(const GemvArgs& A, int mode, bool mixed, int P0, bool bf, int xr, int sub) {
@@ -470,6 +471,11 @@ BStreamPlan plan_bstream(const GemvArgs& A, int dtype, int mode, bool mixed, int
     const bool gateup = mode == CBK_MODE_GATEUP;
     const int64_t U = ceil_div(A.C, 4);
     const int sub = bstream_sub(A.gs);
+    // Below about two million codes a call with finer groups stays on the fp32 matrix-core kernel,
+    // which has no activations to stage (W3, us, that kernel / this one: 512 -> 300 batch 8 6.4 /
+    // 8.4 .. 9.0, 300 -> 5000 5.8 .. 6.4 / 5.3 .. 7.7; 2560 -> 1000 batch 8 fp16 10.1 / 8.3,
+    // 4096^2 18.4 / 8.4, 14336 -> 512 53 / 10).
+    if (sub > 1 && (int64_t)A.V * A.K < BSTREAM_FINE_CODES) return bp;
     bp = bstream_base(A.M, A.C, split_k, gateup, bf, xr, sub);
     if (bstream_fills(bp, A.V)) {
         BStreamPlan fill = bstream_fill(A, mode, mixed, std::max(split_k, 1), bf, xr, sub);

@@ -535,8 +535,9 @@ __device__ __forceinline__ void stream_tail(const GemvArgs& A, char* lds) {
 // == 0).  Groups of multiples of 64 or 32 codes (SUB = 2 or 4) take the unit's 4 / SUB chunks of
 // each sub-unit apart: the MFMAs of a sub-unit see zero codes in the other chunks' lanes (16
 // v_and and 4 MFMAs a sub-unit), and X, XB, scale and zero are per sub-unit.  It is still bound
-// by the stream's latency chains, not by those (W4 g = 64 2560 -> 10240 batch 5: 22.7 us on the
-// fp32 matrix-core kernel, whose loads are a word a lane).  The MFMA sums over k, so no cross-lane reduction is
+// by the stream's latency chains, not by those (W3 batch 8, us: 4096^2 g = 64 18.4 on the fp32
+// matrix-core kernel, whose loads are a word a lane, 8.4 here, g = 32 18.0 and 9.3; 14336 -> 512
+// 53 and 10).  The MFMA sums over k, so no cross-lane reduction is
 // needed; lane (j, kq) holds batch rows 4 kq .. 4 kq + 3 of row j.  Gate-up rows
 // alternate between the waves of a workgroup (even waves gate, odd waves up, the
 // same 16 pair rows), so every wave's rows lie in one projection and its buffer
@@ -722,7 +723,9 @@ __device__ __forceinline__ void bstream_body(const GemvArgs& A, char* lds) {
 #pragma unroll
             for (int q = 0; q < 16; ++q) h[q] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, h[q]) - off);
         }
-#pragma unroll
+        // a loop for SUB > 1: unrolled, the sub-units' LDS reads and masked codes are all live at
+        // once and 130 registers spill (SUB = 4: 26 us instead of 7 at 4096^2)
+#pragma unroll 1
         for (int sub = 0; sub < SUB; ++sub) {
             const int n = uj * SUB + sub;
             const f4 X4 = *reinterpret_cast<const f4*>(XSu + n * 16 + 4 * kq);
@@ -737,9 +740,9 @@ __device__ __forceinline__ void bstream_body(const GemvArgs& A, char* lds) {
                                                            *reinterpret_cast<const h8*>(&bw), d, 0, 0, 0);
             }
             // the sub-unit's scale and zero sit in lane (j, its index % 4), set index / 4
-            const int own = u * SUB + sub;
-            const uint32_t su = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * (j + 16 * (own & 3)), (int)s_own[own >> 2]);
-            const uint32_t zu = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * (j + 16 * (own & 3)), (int)z_own[own >> 2]);
+            const int own = 4 * (j + 16 * ((u * SUB + sub) & 3)), set = u * SUB >> 2;
+            const uint32_t su = (uint32_t)__builtin_amdgcn_ds_bpermute(own, (int)s_own[set]);
+            const uint32_t zu = (uint32_t)__builtin_amdgcn_ds_bpermute(own, (int)z_own[set]);
             const float sc = meta_f<DT>(su);
             const float ze = meta_f<DT>(zu);
             if constexpr (DT != DT_F16) {
