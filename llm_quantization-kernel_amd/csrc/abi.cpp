@@ -403,7 +403,6 @@ BStreamPlan bstream_make(const GemvArgs& A, int mode, bool mixed, int P, int bsu
 // groups); 4096^2 batch 16 10.1 -> 8.9 (P = 2).  The target is a constant -- the CU count
 // of every gfx950 part -- so cbk_gemv_partial_floats can bound P without a device.
 constexpr int BSTREAM_CU_TARGET = 256;
-constexpr int64_t BSTREAM_FINE_CODES = 1 << 21;
 constexpr int BSTREAM_FILL_SPLITS = 4;
 
 BStreamPlan bstream_fill(const GemvArgs& A, int mode, bool mixed, int P0, bool bf, int xr, int sub) {
@@ -450,6 +449,24 @@ bool bstream_fills(const BStreamPlan& base, int64_t V) {
     return base.P > 1 || ceil_div(V, 16 * base.rw) * base.P * 2 <= BSTREAM_CU_TARGET;
 }
 
+// The shortest K at which a call with groups finer than a unit leaves the fp32 matrix-core kernel.
+// That kernel has no activations to stage and no splits, and its time follows K: 5 us at 512, 8 at
+// 2048, 12 at 2560, 17 at 4096 up to 4096 rows, in proportion to the rows past that.  The sub-unit
+// builds cost 4.5 .. 7 us where one split's row blocks cover half the CUs (V > 2048, or 4096 with
+// the two row groups of more than 10 operand rows), else 7 (3 operand rows) to 13 (16) for the
+// splits, hardly more with K.  So the line is low with enough rows (16-bit x; fp32 x at batch 2
+// stages more) and otherwise lies where the other kernel passes the splits' cost.  Measured over
+// 784 points (K 512 .. 4096, V 512 .. 14336, batch 2 .. 16, g = 32 and 64), us, that kernel / this
+// one: fp16 batch 3 V 4096 K 1024 6.2 / 4.6; V 1024 K 2048 7.6 / 7.7, K 2560 8.8 / 7.7; batch 16
+// V 4096 K 2088 8.5 / 11.2, K 3072 13.8 / 11.7; V 8192 K 1024 9.8 / 7.0, K 512 6.6 / 6.5; fp32
+// batch 8 V 8192 K 2088 14.1 / 21.5, K 3072 25.8 / 23.8.
+int bstream_fine_k(int64_t rows, int64_t V, int dtype) {
+    const bool full = V > (rows <= 10 ? 2048 : 4096);
+    if (full && dtype != CBK_F32) return 1024;
+    if (full && rows <= 4) return 1536;
+    return rows <= 10 ? 2560 : 3072;
+}
+
 BStreamPlan plan_bstream(const GemvArgs& A, int dtype, int mode, bool mixed, int split_k, int cus) {
     BStreamPlan bp;
     const int64_t lim = INT32_MAX;
@@ -471,11 +488,7 @@ BStreamPlan plan_bstream(const GemvArgs& A, int dtype, int mode, bool mixed, int
     const bool gateup = mode == CBK_MODE_GATEUP;
     const int64_t U = ceil_div(A.C, 4);
     const int sub = bstream_sub(A.gs);
-    // Below about two million codes a call with finer groups stays on the fp32 matrix-core kernel,
-    // which has no activations to stage (W3, us, that kernel / this one: 512 -> 300 batch 8 6.4 /
-    // 8.4 .. 9.0, 300 -> 5000 5.8 .. 6.4 / 5.3 .. 7.7; 2560 -> 1000 batch 8 fp16 10.1 / 8.3,
-    // 4096^2 18.4 / 8.4, 14336 -> 512 53 / 10).
-    if (sub > 1 && (int64_t)A.V * A.K < BSTREAM_FINE_CODES) return bp;
+    if (sub > 1 && A.K < bstream_fine_k(A.M * xr, A.V, dtype)) return bp;
     bp = bstream_base(A.M, A.C, split_k, gateup, bf, xr, sub);
     if (bstream_fills(bp, A.V)) {
         BStreamPlan fill = bstream_fill(A, mode, mixed, std::max(split_k, 1), bf, xr, sub);

@@ -534,7 +534,10 @@ __device__ __forceinline__ void stream_tail(const GemvArgs& A, char* lds) {
 // with X = sum x and XB = sum x B(k) over the unit (SUB = 1: a unit lies in one group, g % 128
 // == 0).  Groups of multiples of 64 or 32 codes (SUB = 2 or 4) take the unit's 4 / SUB chunks of
 // each sub-unit apart: the MFMAs of a sub-unit see zero codes in the other chunks' lanes (16
-// v_and and 4 MFMAs a sub-unit), and X, XB, scale and zero are per sub-unit.  It is still bound
+// v_and and 4 MFMAs a sub-unit), and X, XB, scale and zero are per sub-unit.  The decoded pairs
+// also lose their 1024 there (16 v_pk_add_f16 a unit), which keeps the error that the fp32
+// products had: fp16 against 64 bits 2.19e-4 with the offset, 2.07e-4 without (W2 11008 -> 4096),
+// at the same speed.  It is still bound
 // by the stream's latency chains, not by those (W3 batch 8, us: 4096^2 g = 64 18.4 on the fp32
 // matrix-core kernel, whose loads are a word a lane, 8.4 here, g = 32 18.0 and 9.3; 14336 -> 512
 // 53 and 10).  The MFMA sums over k, so no cross-lane reduction is
@@ -586,6 +589,9 @@ __device__ __forceinline__ void bstream_body(const GemvArgs& A, char* lds) {
     // them only
     constexpr int XE = DT == DT_F32 ? 4 : 2;           // bytes of an activation / scale / zero
     constexpr int OPR = DT == DT_F32 ? 2 : 1;          // operand rows per batch row (fp32: hi, lo)
+    // The decoded pairs lose their 1024 (exact), so no 1024 sum x cancels in the fp32 sums: for
+    // fp32 x, and for the finer groups, whose calls took fp32 products before.
+    constexpr bool DROP = DT == DT_F32 || SUB > 1;
     const int MR = OPR * M;                            // staged operand rows (<= 16)
     const __amdgpu_buffer_rsrc_t xr =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(A.x), (short)0, A.M * A.K * XE, RAW);
@@ -634,8 +640,8 @@ __device__ __forceinline__ void bstream_body(const GemvArgs& A, char* lds) {
     // per sub-unit n and operand row its sums X (at XSu[n * 16 + o]) and XB (XBu[n * 16 + o]), and
     // for bf16 and fp32 the unit's prescale 2^c (XFu[u * 16 + o]; the four chunks of a unit
     // share c, from their largest exponent, since the MFMA sums over the unit).  Operand row o
-    // is batch row o, or for fp32 half o & 1 (hi, lo) of batch row o >> 1, whose decoded
-    // pairs lose their 1024 (XB = 0).
+    // is batch row o, or for fp32 half o & 1 (hi, lo) of batch row o >> 1.  XB is left out
+    // with DROP.
     u4* Xl = reinterpret_cast<u4*>(lds);
     float* XSu = reinterpret_cast<float*>(lds + 64 * NCH * MR);
     float* XBu = XSu + 16 * SUB * NU;
@@ -666,8 +672,6 @@ __device__ __forceinline__ void bstream_body(const GemvArgs& A, char* lds) {
             if (c % SCH == 0) {
                 XSu[c / SCH * 16 + 2 * i] = xsh;
                 XSu[c / SCH * 16 + 2 * i + 1] = xso;
-                XBu[c / SCH * 16 + 2 * i] = 0.f;
-                XBu[c / SCH * 16 + 2 * i + 1] = 0.f;
             }
             if ((c & 3) == 0) {
                 const float f = __builtin_ldexpf(1.0f, cu);
@@ -692,12 +696,12 @@ __device__ __forceinline__ void bstream_body(const GemvArgs& A, char* lds) {
             // the 4 chunks of a unit are 4 consecutive threads (NCH % 4 == 0)
 #pragma unroll
             for (int o = 1; o < SCH; o *= 2) {
-                B += __shfl_xor(B, o, 64);
+                if constexpr (!DROP) B += __shfl_xor(B, o, 64);
                 xs += __shfl_xor(xs, o, 64);
             }
             if (c % SCH == 0) {
                 XSu[c / SCH * 16 + i] = xs;
-                XBu[c / SCH * 16 + i] = B;
+                if constexpr (!DROP) XBu[c / SCH * 16 + i] = B;
             }
             if constexpr (DT == DT_BF16)
                 if ((c & 3) == 0) XFu[(c >> 2) * 16 + i] = __builtin_ldexpf(1.0f, cu);
@@ -718,7 +722,7 @@ __device__ __forceinline__ void bstream_body(const GemvArgs& A, char* lds) {
         for (int m = 0; m < 4; ++m) a[m] = Xl[(m * NCH + c) * MR + ia];
         uint32_t h[16];
         Decode<BITS>::run(w[u], h, g);
-        if constexpr (DT == DT_F32) {
+        if constexpr (DROP) {
             const h2 off = {(_Float16)1024.f, (_Float16)1024.f};
 #pragma unroll
             for (int q = 0; q < 16; ++q) h[q] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, h[q]) - off);
@@ -729,7 +733,8 @@ __device__ __forceinline__ void bstream_body(const GemvArgs& A, char* lds) {
         for (int sub = 0; sub < SUB; ++sub) {
             const int n = uj * SUB + sub;
             const f4 X4 = *reinterpret_cast<const f4*>(XSu + n * 16 + 4 * kq);
-            const f4 XB4 = *reinterpret_cast<const f4*>(XBu + n * 16 + 4 * kq);
+            f4 XB4 = {0.f, 0.f, 0.f, 0.f};
+            if constexpr (!DROP) XB4 = *reinterpret_cast<const f4*>(XBu + n * 16 + 4 * kq);
             // the lanes whose chunk is outside the sub-unit hold zeros
             const uint32_t in = SUB == 1 || kq / SCH == sub ? 0xFFFFFFFFu : 0u;
             f4 d = {0.f, 0.f, 0.f, 0.f};

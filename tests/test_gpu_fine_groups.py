@@ -1,6 +1,6 @@
 """Batched decode with groups finer than 128 codes on the streaming kernel's sub-unit builds
-(multiples of 64, and of 32), against the oracle.  The last shape is one of the small calls that
-stay on the fp32 matrix-core kernel.
+(multiples of 64, and of 32), against the oracle.  The shapes lie on both sides of the line
+below which a call stays on the fp32 matrix-core kernel (K against rows and batch).
 
 The bars: one output rounding (2^-11 fp16, 2^-8 bf16) of the largest output plus 1e-4 for the fp32
 sums and the operands' staging; fp32 1e-6, four times the kernel's error against 64 bits."""
@@ -43,7 +43,7 @@ def off(y, ref):
 @pytest.mark.parametrize("bits", [2, 3, 4])
 @pytest.mark.parametrize("N,K,gs", [(1100, 2048, 64), (2100, 1000, 64), (515, 4128, 32), (3300, 640, 96),
                                     (22001, 96, 32), (520, 4104, 192), (200, 11008, 64), (1100, 2080, 160),
-                                    (300, 512, 64)])
+                                    (300, 512, 64), (4500, 1160, 64), (4500, 3112, 96), (2100, 1568, 32)])
 def test_fine_groups(hip, dtype, M, bits, N, K, gs):
     w, W, b = make(N, K, bits, dtype, gs, bias=True)
     x = randx(M, K, dtype)
@@ -105,3 +105,16 @@ def test_fine_groups_at_the_scratch_limit(hip):
     assert rc == 0, cabi.last_error()
     torch.cuda.synchronize()
     assert off(out, y.double().cpu().numpy()) < 2 * BAR[torch.float16]      # two results, a rounding each
+
+
+@pytest.mark.parametrize("gs", [32, 64])
+def test_fine_groups_fp16_error(hip, gs):
+    """The 16-bit builds keep the precision of fp32 products: against 64 bits, no more than 1 % over
+    the error of rounding the exact result to fp16 once (in quadrature, 3e-5 of other error).  With
+    1024 left in the decoded pairs it is 5 % over."""
+    M, N, K = 5, 4096, 11008
+    w, W, _ = make(N, K, 2, torch.float16, gs)
+    x = randx(M, K, torch.float16)
+    ref = torch.from_numpy(x.double().cpu().numpy() @ W.T)
+    once = (ref.half().double() - ref).norm()
+    assert (packed_linear(x, w).double().cpu() - ref).norm() < 1.01 * once
