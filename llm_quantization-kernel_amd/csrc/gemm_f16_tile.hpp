@@ -21,7 +21,8 @@
 // Load group t holds the wave's eighth of activation stage t + 2 (128 rows x 128
 // codes, XOR-swizzled 16-byte pieces, into a ring of three stage slots) and, at
 // even t, of weight block t / 2 + 1 (256 codes of the tile's 128 packed rows,
-// double-buffered) and of a scale / zero window (8 groups per row).  Group t's
+// double-buffered) and, where the block starts one, of a scale / zero window (8 groups
+// per row).  Group t's
 // instructions go out in eight slots, two per k-step, between barrier t and the
 // wait before barrier t + 1, so no wave stalls long on a full memory queue while
 // the MFMAs starve.  Before barrier t + 1 a wave waits until at most group t is in
