@@ -130,13 +130,15 @@ hipError_t scratch_for(int device, float** out) {
 // has one holder for good:
 //  * a stream, for its eager calls -- calls on one stream run in order, so one window
 //    serves all of them;
-//  * a graph capture -- the captured launches keep the window's address and may be
-//    replayed at any time on any stream, so the window is never handed to eager calls
-//    or to another capture.
+//  * a stream within a graph capture -- the captured launches keep the window's address
+//    and may be replayed at any time on any stream, so the window is never handed to
+//    eager calls or to another capture; and of the streams forked into one capture each
+//    has its own, because their launches become parallel branches of the graph.
 // A window is never taken from its holder (a stream may still have split calls in
 // flight).  A call that finds no window of its own and no free one, or whose row blocks
 // outnumber a window's counters, takes the combine launch instead: correct, one launch
-// more.  One graph must not be replayed while another replay of it runs.
+// more.  So does a call on hipStreamPerThread, one handle for a stream of each thread.
+// One graph must not be replayed while another replay of it runs.
 constexpr int SPLIT_WINDOWS = 256;
 constexpr int SPLIT_COUNTERS = 4096;
 static __device__ __align__(256) uint32_t split_counters[SPLIT_WINDOWS * SPLIT_COUNTERS];
@@ -148,14 +150,14 @@ struct SplitWindows {
     bool init = false;
     int used = 0;                                   // windows [0, used) have holders
     bool by_capture[SPLIT_WINDOWS];
-    hipStream_t stream[SPLIT_WINDOWS];              // holder stream (eager windows)
-    unsigned long long capture[SPLIT_WINDOWS];      // holder capture id (capture windows)
+    hipStream_t stream[SPLIT_WINDOWS];              // holder stream
+    unsigned long long capture[SPLIT_WINDOWS];      // and its capture's id (capture windows)
 };
 SplitWindows g_split[MAX_DEVICES];
 
 // The counter window of this call on `device` (made current by the caller), or nullptr.
 uint32_t* split_window(int device, hipStream_t stream) {
-    if (device < 0 || device >= MAX_DEVICES) return nullptr;
+    if (device < 0 || device >= MAX_DEVICES || stream == hipStreamPerThread) return nullptr;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     unsigned long long id = 0;
     if (hipStreamGetCaptureInfo(stream, &st, &id) != hipSuccess) return nullptr;
@@ -171,12 +173,12 @@ uint32_t* split_window(int device, hipStream_t stream) {
     if (!W.base) return nullptr;
     int slot = -1;
     for (int i = 0; i < W.used && slot < 0; ++i)
-        if (W.by_capture[i] == cap && (cap ? W.capture[i] == id : W.stream[i] == stream)) slot = i;
+        if (W.by_capture[i] == cap && W.stream[i] == stream && (!cap || W.capture[i] == id)) slot = i;
     if (slot < 0) {
         if (W.used == SPLIT_WINDOWS) return nullptr;
         slot = W.used++;
         W.by_capture[slot] = cap;
-        W.stream[slot] = cap ? nullptr : stream;
+        W.stream[slot] = stream;
         W.capture[slot] = cap ? id : 0;
     }
     return W.base + (size_t)slot * SPLIT_COUNTERS;

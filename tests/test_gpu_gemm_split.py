@@ -124,3 +124,42 @@ def test_split_gemm_streams_and_replays(hip):
         first = yg.clone() if first is None else first
         assert torch.equal(yg, first)
     assert off(first, ref) < BAR[torch.float16]
+
+
+def test_split_calls_on_forked_capture_streams(hip):
+    """Split calls on streams forked into one capture become parallel branches of its graph, so each
+    branch needs arrival counters of its own: every replay, between eager calls, gives the eager
+    bits, for prefill GEMMs and decode calls alike."""
+    shapes = [(512, 40, 4096), (256, 8, 11008), (384, 40, 4096), (320, 8, 11008), (512, 33, 5120), (384, 8, 11008)]
+    calls = []
+    for i, (N, M, K) in enumerate(shapes):                 # a prefill and a decode call for each branch
+        if M > 16:
+            assert splits(M, N, K, torch.float16)
+        else:
+            assert _C.decode_plan(torch.float16, M, K, 128, N, 3, "gemv", 1, 1)[1] > 1
+        calls.append((randx(M, K, torch.float16, i), make(N, K, 3, torch.float16, 128, i)[0]))
+    eager = [packed_linear(x, w) for x, w in calls]
+    torch.cuda.synchronize()
+    sides = [torch.cuda.Stream(), torch.cuda.Stream()]
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        main = torch.cuda.current_stream()
+        outs = []
+        for i, st in enumerate((main, *sides)):
+            if st is not main:
+                st.wait_stream(main)
+            with torch.cuda.stream(st):
+                outs += [[packed_linear(x, w) for _ in range(4)] for x, w in calls[2 * i:2 * i + 2]]
+        for st in sides:
+            main.wait_stream(st)
+    for _ in range(5):
+        for o in outs:
+            for t in o:
+                t.zero_()
+        g.replay()
+        again = [packed_linear(x, w) for x, w in calls]
+        torch.cuda.synchronize()
+        for o, y, z in zip(outs, eager, again):
+            assert torch.equal(z, y)
+            for t in o:
+                assert torch.equal(t, y)
