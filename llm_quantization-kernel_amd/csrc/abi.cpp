@@ -138,10 +138,13 @@ hipError_t scratch_for(int device, float** out) {
 // flight).  A call that finds no window of its own and no free one, or whose row blocks
 // outnumber a window's counters, takes the combine launch instead: correct, one launch
 // more.  So does a call on hipStreamPerThread, one handle for a stream of each thread.
-// One graph must not be replayed while another replay of it runs.
+// One graph must not be replayed while another replay of it runs.  Decode calls and
+// prefill GEMMs have windows of their own (WIN_DECODE, WIN_GEMM): a program that captures
+// a graph per prompt length leaves its decode graphs theirs.
+enum { WIN_DECODE = 0, WIN_GEMM = 1 };
 constexpr int SPLIT_WINDOWS = 256;
 constexpr int SPLIT_COUNTERS = 4096;
-static __device__ __align__(256) uint32_t split_counters[SPLIT_WINDOWS * SPLIT_COUNTERS];
+static __device__ __align__(256) uint32_t split_counters[2 * SPLIT_WINDOWS * SPLIT_COUNTERS];
 
 struct SplitWindows {
     std::mutex mu;
@@ -153,21 +156,23 @@ struct SplitWindows {
     hipStream_t stream[SPLIT_WINDOWS];              // holder stream
     unsigned long long capture[SPLIT_WINDOWS];      // and its capture's id (capture windows)
 };
-SplitWindows g_split[MAX_DEVICES];
+SplitWindows g_split[2][MAX_DEVICES];
 
 // The counter window of this call on `device` (made current by the caller), or nullptr.
-uint32_t* split_window(int device, hipStream_t stream) {
+// kind: WIN_DECODE or WIN_GEMM.
+uint32_t* split_window(int kind, int device, hipStream_t stream) {
     if (device < 0 || device >= MAX_DEVICES || stream == hipStreamPerThread) return nullptr;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     unsigned long long id = 0;
     if (hipStreamGetCaptureInfo(stream, &st, &id) != hipSuccess) return nullptr;
     const bool cap = st == hipStreamCaptureStatusActive;
-    SplitWindows& W = g_split[device];
+    SplitWindows& W = g_split[kind][device];
     std::lock_guard<std::mutex> lk(W.mu);
     if (!W.init) {
         void* p = nullptr;
         W.err = hipGetSymbolAddress(&p, HIP_SYMBOL(split_counters));
-        W.base = W.err == hipSuccess ? static_cast<uint32_t*>(p) : nullptr;
+        W.base = W.err == hipSuccess ? static_cast<uint32_t*>(p) + (size_t)kind * SPLIT_WINDOWS * SPLIT_COUNTERS
+                                     : nullptr;
         W.init = true;
     }
     if (!W.base) return nullptr;
@@ -641,7 +646,7 @@ int run_decode(GemvArgs& A, int dtype, int mode, bool mixed, int split_k, int rh
     if (A.P > 1) {
         if (!partial) return fail(CBK_EINVAL, "split-K needs a partial buffer (cbk_gemv_partial_floats)");
         A.partial = partial;
-        if (combines_in_dispatch(L)) A.split_cnt = split_window(device, s);
+        if (combines_in_dispatch(L)) A.split_cnt = split_window(WIN_DECODE, device, s);
     } else {
         A.partial = nullptr;
     }
@@ -747,7 +752,7 @@ GemmPlan plan_gemm_f16(GemmArgs& A, int64_t ntiles, float* partial, int64_t part
     if (p.S > 1 && (!partial || partial_floats < p.partial_floats)) p = gemm_f16_plan(A.M, ntiles, A.K, false);
     A.S = p.S;
     A.partial = p.S > 1 ? partial : nullptr;
-    A.split_cnt = p.S > 1 && p.tiles <= SPLIT_COUNTERS ? split_window(device, s) : nullptr;
+    A.split_cnt = p.S > 1 && p.tiles <= SPLIT_COUNTERS ? split_window(WIN_GEMM, device, s) : nullptr;
     return p;
 }
 
