@@ -8,7 +8,9 @@
 // that meets half slot p is staged as x * 2^-e(p) in fp16 (a power-of-two scale: exact
 // while the product stays a normal fp16, |x| 2^-e >= 2^-14; below that it rounds to a
 // subnormal and keeps fewer bits), so the MFMA sums x * (B(p) + q) with the slot offset
-// B(p) = 2^(10 - e(p)); the kernels remove sum_p x * B(p) together with the zero point.
+// B(p) = 2^(10 - e(p)); the kernels remove sum_p x * B(p) together with the zero point, or
+// (builds that must not lose those bits) the offset or the whole of 2^e and B from the decoded
+// pair before the product.
 //
 // Half slot p (pair p >> 1, high half when p & 1) holds code kappa(p) at offset
 // expo(p).  MFMA operand m (8 halves) is pairs 4m .. 4m+3.  Each output pair is

@@ -105,8 +105,10 @@ __device__ __forceinline__ void load_x(__amdgpu_buffer_rsrc_t xr, bool ok, int b
     }
 }
 
-// Operand pairs of one chunk for the BITS decode, their slot-offset sum B and sum x.
-template <int BITS>
+// Operand pairs of one chunk for the BITS decode, their slot-offset sum B and sum x.  !SCALED: the
+// pairs are the activations as they are, for decoded pairs that hold the codes themselves (B is
+// of no use then).
+template <int BITS, bool SCALED = true>
 __device__ __forceinline__ void convert_x(const uint32_t (&x)[16], u4 (&X)[4], float& B, float& xs) {
     const h2 one = {(_Float16)1.0f, (_Float16)1.0f};
     uint32_t o[16];
@@ -120,7 +122,8 @@ __device__ __forceinline__ void convert_x(const uint32_t (&x)[16], u4 (&X)[4], f
                              ((uint32_t)(4 + 2 * (kb & 1)) << 16) | ((uint32_t)(5 + 2 * (kb & 1)) << 24);
         const uint32_t raw = __builtin_amdgcn_perm(x[kb >> 1], x[ka >> 1], sel);
         const h2 sc = {(_Float16)(1.0f / (float)(1 << ea)), (_Float16)(1.0f / (float)(1 << eb))};
-        const h2 v = __builtin_bit_cast(h2, raw) * sc;      // power-of-two scale: exact unless subnormal
+        h2 v = __builtin_bit_cast(h2, raw);
+        if constexpr (SCALED) v = v * sc;                   // power-of-two scale: exact unless subnormal
         o[p] = __builtin_bit_cast(uint32_t, v);
         b = __builtin_amdgcn_fdot2(v, one, b, false);
         t = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, x[p]), one, t, false);
@@ -535,9 +538,11 @@ __device__ __forceinline__ void stream_tail(const GemvArgs& A, char* lds) {
 // == 0).  Groups of multiples of 64 or 32 codes (SUB = 2 or 4) take the unit's 4 / SUB chunks of
 // each sub-unit apart: the MFMAs of a sub-unit see zero codes in the other chunks' lanes (16
 // v_and and 4 MFMAs a sub-unit), and X, XB, scale and zero are per sub-unit.  The decoded pairs
-// also lose their 1024 there (16 v_pk_add_f16 a unit), which keeps the error that the fp32
-// products had: fp16 against 64 bits 2.19e-4 with the offset, 2.07e-4 without (W2 11008 -> 4096),
-// at the same speed.  It is still bound
+// also lose their 1024 there, and for fp16 x their 2^e (16 v_pk_add_f16 or v_pk_fma_f16 a unit),
+// which keeps the error that the fp32 products had at every magnitude of x, at the same speed.
+// fp16 against 64 bits: W2 11008 -> 4096 at unit scale 2.19e-4 with the offset, 2.07e-4 without; W3
+// 4096^2 at an rms of 1e-3 / 1e-4 / 1e-5 7.8e-4 / 4.0e-3 / 4.4e-2 with x staged times 2^-e, 2.1e-4 /
+// 2.2e-4 / 1.3e-3 (subnormal outputs) without, as on the fp32 matrix-core kernel.  It is still bound
 // by the stream's latency chains, not by those (W3 batch 8, us: 4096^2 g = 64 18.4 on the fp32
 // matrix-core kernel, whose loads are a word a lane, 8.4 here, g = 32 18.0 and 9.3; 14336 -> 512
 // 53 and 10).  The MFMA sums over k, so no cross-lane reduction is
@@ -590,8 +595,11 @@ __device__ __forceinline__ void bstream_body(const GemvArgs& A, char* lds) {
     constexpr int XE = DT == DT_F32 ? 4 : 2;           // bytes of an activation / scale / zero
     constexpr int OPR = DT == DT_F32 ? 2 : 1;          // operand rows per batch row (fp32: hi, lo)
     // The decoded pairs lose their 1024 (exact), so no 1024 sum x cancels in the fp32 sums: for
-    // fp32 x, and for the finer groups, whose calls took fp32 products before.
+    // fp32 x, and for the finer groups, whose calls took fp32 products before.  For those in fp16
+    // they lose their slot scale 2^e too (RAWQ, the same instruction), so that the activations are
+    // staged as they are: times 2^-e they would round from 2^-9 down.
     constexpr bool DROP = DT == DT_F32 || SUB > 1;
+    constexpr bool RAWQ = DT == DT_F16 && SUB > 1;
     const int MR = OPR * M;                            // staged operand rows (<= 16)
     const __amdgpu_buffer_rsrc_t xr =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(A.x), (short)0, A.M * A.K * XE, RAW);
@@ -689,7 +697,7 @@ __device__ __forceinline__ void bstream_body(const GemvArgs& A, char* lds) {
                 cu = prescale_bf16(E);
                 convert_x_bf16_at<BITS>(xa[e], cu, X, B, xs);
             } else {
-                convert_x<BITS>(xa[e], X, B, xs);
+                convert_x<BITS, !RAWQ>(xa[e], X, B, xs);
             }
 #pragma unroll
             for (int m = 0; m < 4; ++m) Xl[(m * NCH + c) * M + i] = X[m];
@@ -722,7 +730,15 @@ __device__ __forceinline__ void bstream_body(const GemvArgs& A, char* lds) {
         for (int m = 0; m < 4; ++m) a[m] = Xl[(m * NCH + c) * MR + ia];
         uint32_t h[16];
         Decode<BITS>::run(w[u], h, g);
-        if constexpr (DROP) {
+        if constexpr (RAWQ) {
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const float fa = 1.f / (float)(1 << Decode<BITS>::expo(2 * q));
+                const float fb = 1.f / (float)(1 << Decode<BITS>::expo(2 * q + 1));
+                const h2 m = {(_Float16)fa, (_Float16)fb}, o = {(_Float16)(-1024.f * fa), (_Float16)(-1024.f * fb)};
+                h[q] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2, h[q]), m, o));
+            }
+        } else if constexpr (DROP) {
             const h2 off = {(_Float16)1024.f, (_Float16)1024.f};
 #pragma unroll
             for (int q = 0; q < 16; ++q) h[q] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, h[q]) - off);
