@@ -591,6 +591,7 @@ DecodeLaunch plan_decode(GemvArgs& A, int dtype, int mode, bool mixed, int split
         A.divP = make_fastdiv((uint32_t)A.P);
         A.divRW = make_fastdiv((uint32_t)A.st_rw);
         A.divG = make_fastdiv((uint32_t)(A.gs * bp.sub / 128));
+        A.divGS = make_fastdiv((uint32_t)(A.gs / 32));
         // the builds for finer groups count as the generic family: the calls that the 128-code
         // units do not take
         L.family = bp.sub == 1 ? CBK_KERNEL_BSTREAM : CBK_KERNEL_GENERIC;

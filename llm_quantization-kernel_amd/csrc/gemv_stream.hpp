@@ -551,6 +551,44 @@ __device__ __forceinline__ void stream_tail(const GemvArgs& A, char* lds) {
 // same 16 pair rows), so every wave's rows lie in one projection and its buffer
 // descriptors stay uniform.
 
+// The products of virtual row v with batch row i over chunks [ca, cb), one by one as the fp32
+// matrix-core kernel forms them: (q - z) s first.  The sub-unit builds take a sum from here where
+// theirs is not finite -- they multiply an infinite activation by the zero codes of the other
+// sub-units and subtract z sum x, so it would leave NaN where its products are infinities of one
+// sign, and z sum x or the scaled-back sum may overflow where (q - z) s x does not.  No hurry here:
+// a loop over single codes.  The look at the sums costs 0.3 % (80 points in the geometric mean).
+template <int BITS, int MODE, int DT>
+__device__ __forceinline__ float plain_sum(const GemvArgs& A, int v, int i, int ca, int cb) {
+    int proj, r;
+    vmap<MODE>(A, v, proj, r);
+    const Src& S = A.src[proj];
+    const uint32_t* row = S.w + (long)r * S.wpr;
+    float acc = 0.f, s = 0.f, nzs = 0.f;
+#pragma unroll 1
+    for (int k = 32 * ca; k < min(32 * cb, A.K); ++k) {
+        const int c = k >> 5, bit = (k & 31) * BITS;
+        if ((k & 31) == 0) {
+            const long g = (long)r * A.G + (int)fdiv((uint32_t)c, A.divGS);
+            s = load_f<DT>(S.s, g);
+            nzs = -load_f<DT>(S.z, g) * s;
+        }
+        const uint32_t* w = row + (long)c * BITS + (bit >> 5);
+        const uint32_t hi = (bit & 31) + BITS > 32 ? w[1] : 0u;
+        const uint32_t q = (uint32_t)((((uint64_t)hi << 32) | w[0]) >> (bit & 31)) & ((1u << BITS) - 1u);
+        acc = fmaf(load_f<DT>(A.x, (long)i * A.K + k), fmaf((float)q, s, nzs), acc);
+    }
+    return acc;
+}
+
+// The kernel's arguments read anew (GemvArgs is the batched kernel's only one), by a pointer the
+// compiler cannot see through: what only a rare path reads is then not held in registers for it (72
+// SGPRs instead of 65 in the plain W4 build), or loaded at the kernel's start.
+__device__ __forceinline__ const GemvArgs& args_again() {
+    const void* p = (const void*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *reinterpret_cast<const GemvArgs*>(p);
+}
+
 template <int BITS, int MODE, int BSU, int DT, int SUB>
 __device__ __forceinline__ void bstream_body(const GemvArgs& A, char* lds) {
     const int tid = threadIdx.x, lane = tid & 63;
@@ -779,17 +817,29 @@ __device__ __forceinline__ void bstream_body(const GemvArgs& A, char* lds) {
 
     // 4. row totals per slice: lane (j, kq) holds operand rows 4 kq + q of row j (fp32: the
     // hi and lo rows of batch rows 2 kq and 2 kq + 1)
-    if constexpr (DT == DT_F32) {
+    constexpr int NR = 4 / OPR;                   // the lane's batch rows (past M: unset sums)
+    float mag = 0.f;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int i = 2 * kq + h;
-            if (i < M) red[(ks * M + i) * RB + roff] = acc[2 * h] + acc[2 * h + 1];
+    for (int h = 0; h < NR; ++h) {
+        const int i = NR * kq + h;
+        const float y = DT == DT_F32 ? acc[2 * h] + acc[2 * h + 1] : acc[h];
+        if (i < M) {
+            red[(ks * M + i) * RB + roff] = y;
+            mag += fabsf(y);
         }
-    } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int i = 4 * kq + q;
-            if (i < M) red[(ks * M + i) * RB + roff] = acc[q];
+    }
+    if constexpr (SUB > 1) {
+        // a sum that is not finite (infinities and NaNs in the inputs leave no other) is formed again
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!__builtin_isfinite(mag)) != 0, 0)) {
+            const GemvArgs& B = args_again();
+            const int bu0 = (int)fdiv((uint32_t)(((B.C + 3) >> 2) * p), B.divP);
+            const int bu1 = (int)fdiv((uint32_t)(((B.C + 3) >> 2) * (p + 1)), B.divP);
+            const int ca = 4 * (bu0 + BSU * ks), cb = min(min(4 * bu1, B.C), ca + 4 * BSU);
+#pragma unroll 1
+            for (int i = NR * kq; vin && i < min(NR * kq + NR, M); ++i) {
+                float* at = red + (ks * M + i) * RB + roff;
+                if (!__builtin_isfinite(*at)) *at = plain_sum<BITS, MODE, DT>(B, vrow, i, ca, cb);
+            }
         }
     }
     lds_barrier();

@@ -137,6 +137,53 @@ def test_fine_groups_magnitudes(hip, dtype, dist, bits, gs, M):
     assert (packed_linear(x, w).double().cpu() - ref).norm() < 1.01 * once
 
 
+def same_specials(y, z, bar):
+    """The infinities and NaNs of z, and finite values within the bar of z's largest."""
+    assert torch.equal(y.isnan(), z.isnan())
+    assert torch.equal(y.isinf(), z.isinf()) and torch.equal(y[y.isinf()], z[z.isinf()])
+    f = z.isfinite()
+    assert f.any()
+    assert (y[f].double() - z[f].double()).abs().max() <= 2 * bar * z[f].double().abs().max()
+
+
+@pytest.mark.parametrize("kind", ["x inf", "x -inf and nan", "x large", "scale inf", "zero inf"])
+@pytest.mark.parametrize("gs,M,K", [(64, 5, 4096), (32, 8, 3080), (96, 4, 11008)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_fine_groups_not_finite(hip, dtype, kind, gs, M, K):
+    """Infinities and NaNs, and activations near the top of the type's range, come out as the fp32
+    matrix-core kernel gives them, which forms (q - z) s first: infinities of one sign stay
+    infinities, sums that fit stay finite, other rows stay as they are.  That kernel takes the
+    same call with x off 16-byte alignment."""
+    ws = [make(n, K, b, dtype, gs, i)[0] for i, (n, b) in enumerate(((1024, 4), (512, 2), (512, 3), (512, 3)))]
+    x = randx(M, K, dtype)
+    if kind == "x inf":
+        x[1, 77] = float("inf")
+        x[M - 1, K - 1] = float("inf")
+    elif kind == "x -inf and nan":
+        x[0, 5] = -float("inf")
+        x[M - 1, 700] = float("nan")
+        x[2, 9], x[2, 2100] = float("inf"), -float("inf")
+    elif kind == "x large":
+        # outputs of rms 0.05 sqrt(K) times this, 5e37, so six of them fit fp32; z sum x over a
+        # sub-unit, 7.5 sqrt(32) times this, does not
+        x[1] *= 1e3 if dtype == torch.float16 else 1e39 / K ** 0.5
+    else:
+        for w in ws:
+            t = w.scales if kind == "scale inf" else w.zeros
+            t[3, K // gs // 2] = float("inf")
+            t[17, 0] = float("inf")
+    off1 = torch.empty(M * K + 1, dtype=dtype, device="cuda")[1:].view(M, K).copy_(x)
+    bar = BAR[dtype]
+    y, z = packed_linear(x, ws[0]), packed_linear(off1, ws[0])
+    same_specials(y, z, bar)
+    assert z.isinf().any() or kind != "x inf"
+    for qkv in (ws[:3], (ws[3], ws[2], ws[3])):            # a width per projection, and one for all
+        for a, b in zip(fused_qkv(x, *qkv), fused_qkv(off1, *qkv)):
+            same_specials(a, b, bar)
+    if kind != "x large":                                  # (the product of two large factors)
+        same_specials(fused_gate_up(x, ws[2], ws[3]), fused_gate_up(off1, ws[2], ws[3]), 3 * bar)
+
+
 @pytest.mark.parametrize("gs", [32, 64])
 def test_fine_groups_fp16_error(hip, gs):
     """The 16-bit builds keep the precision of fp32 products: against 64 bits, no more than 1 % over
