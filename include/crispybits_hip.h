@@ -100,7 +100,8 @@ int cbk_packed_gemv(const void* x, int dtype, int64_t M, int64_t K,
  * loops, harnesses that forbid hipMalloc).  The split-K partial sums live in a file-scope
  * device array of CBK_NOALLOC_PARTIAL_FLOATS fp32 values per GPU (8 MiB, held until the
  * process ends) instead of a caller buffer; calls whose cbk_gemv_partial_floats(...)
- * exceeds that return CBK_EINVAL.  The call allocates nothing (no hipMalloc, no library
+ * exceeds that return CBK_EINVAL (groups finer than 128 codes at batch 3 and up: only those
+ * whose requested splits do; with split_k = 1 such a call does not use the array).  The call allocates nothing (no hipMalloc, no library
  * allocation); every partial it reads it has written in the same call, so nothing needs
  * clearing between calls.  Calls that overlap on one GPU (concurrent streams, threads)
  * share the array and race. */

@@ -898,10 +898,10 @@ int cbk_packed_gemv_noalloc(const void* x, int dtype, int64_t M, int64_t K, cons
     if (split_k < 1) return fail(CBK_EINVAL, "split_k must be >= 1");
     if (act < 0 || act > 2) return fail(CBK_EINVAL, "act must be 0 (none), 1 (relu) or 2 (silu)");
     if (!out) return fail(CBK_EINVAL, "packed_gemv_noalloc: out must be non-null");
-    // fine groups: a plan whose splits outgrow the scratch gives way to the one that needs fewer
-    int64_t need = partial_floats(dtype, M, N, K, group_size, split_k, true);
-    const bool fine = need <= NOALLOC_PARTIAL_FLOATS;
-    if (!fine) need = partial_floats(dtype, M, N, K, group_size, split_k, false);
+    // fine groups: splits that the caller did not ask for stay out of the scratch, which calls that
+    // overlap share -- without a buffer run_decode takes the streaming plan only unsplit
+    const int64_t need = partial_floats(dtype, M, N, K, group_size, split_k, false);
+    const bool fine = need == 0;
     if (need > NOALLOC_PARTIAL_FLOATS)
         return fail(CBK_EINVAL,
                     "packed_gemv_noalloc: split-K partial sums need %lld floats, above the %lld-float device "
