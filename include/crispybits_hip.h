@@ -68,18 +68,21 @@ int cbk_tile_n(void);
  * (replaces crispybits_max_rho_mode, packed_gemv.cu:343-347). */
 int cbk_max_rho(int device, int bits, int mode, int* out);
 
-/* Decode kernel families reported by cbk_decode_plan: the streaming kernel at batch 1-2
- * (fp16 / bf16), the batched streaming kernel at batch 3-16 (fp16 / bf16, group sizes that
- * are multiples of 128), and the fp32 matrix-core kernel for every other call (fp32
- * activations, unaligned x, other group sizes at batch 3-16, batch > 16).  Values 3 and 5
- * named kernels this library no longer has and are not returned. */
+/* Decode kernel families reported by cbk_decode_plan: the streaming kernel (fp16 / bf16 at
+ * batch 1-2, fp32 at batch 1), the batched streaming kernel (fp16 / bf16 at batch 3-16, fp32
+ * at batch 2-8; group sizes that are multiples of 128, and others from a K on that depends on
+ * rows and batch), and the fp32 matrix-core kernel for every other call (K % 8 != 0 or
+ * unaligned x, finer groups at a shorter K, larger batches).  Values 3 and 5 named kernels
+ * this library no longer has and are not returned. */
 enum { CBK_KERNEL_STREAM = 1, CBK_KERNEL_BSTREAM = 2, CBK_KERNEL_MFMA = 3, CBK_KERNEL_GENERIC = 4, CBK_KERNEL_BATCH = 5 };
 
 /* Additive policy query (no counterpart in the reference, whose tuner infers launches from
  * (split_k, rho), autotune.py:55-88): the launch a decode call with these arguments makes,
  * without launching it.  out[6] = {kernel family, K splits, workgroups, threads per workgroup,
  * dynamic LDS bytes, launches per call}.  n1/n2 and bits1/bits2 are read for CBK_MODE_QKV
- * only; tensors are assumed allocated as torch allocates them (aligned bases). */
+ * only; tensors are assumed allocated as torch allocates them (aligned bases), with the partial
+ * buffer of cbk_gemv_partial_floats: without one, calls with groups finer than 128 codes whose
+ * plan has splits take the fp32 matrix-core kernel instead. */
 int cbk_decode_plan(int dtype, int64_t M, int64_t K, int group_size, int64_t n0, int64_t n1, int64_t n2,
                     int bits0, int bits1, int bits2, int mode, int split_k, int rho, int device, int32_t* out);
 

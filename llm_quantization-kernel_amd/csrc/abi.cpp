@@ -592,9 +592,7 @@ DecodeLaunch plan_decode(GemvArgs& A, int dtype, int mode, bool mixed, int split
         A.divRW = make_fastdiv((uint32_t)A.st_rw);
         A.divG = make_fastdiv((uint32_t)(A.gs * bp.sub / 128));
         A.divGS = make_fastdiv((uint32_t)(A.gs / 32));
-        // the builds for finer groups count as the generic family: the calls that the 128-code
-        // units do not take
-        L.family = bp.sub == 1 ? CBK_KERNEL_BSTREAM : CBK_KERNEL_GENERIC;
+        L.family = CBK_KERNEL_BSTREAM;
         L.f = gemv_bstream_kernel_for(mode, A.bits[0], mixed, bp.bsu, dtype, bp.sub);
         L.grid = bp.grid;
         L.block = 64 * bp.ks * bp.rw;

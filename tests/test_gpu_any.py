@@ -26,12 +26,13 @@ def plan(dtype, M, K, gs, out, bits, kind="gemv", split_k=1):
 
 
 def fp32_family(M, K, gs=128):
-    """Decode family of an fp32 call: streaming at batch 1, the batched streaming kernel at
-    batch 2..8 (two operand rows per batch row, 16 at most; groups of whole 128-code units), the
-    fp32 matrix-core kernel otherwise."""
+    """Decode family of an fp32 call of a few hundred rows: streaming at batch 1, the batched
+    streaming kernel at batch 2..8 (two operand rows per batch row, 16 at most; groups of whole
+    128-code units, and finer ones from K = 2560 on, 3072 above batch 5), the fp32 matrix-core
+    kernel otherwise."""
     if M == 1:
         return "stream"
-    return "bstream" if 2 <= M <= 8 and gs % 128 == 0 else "generic"
+    return "bstream" if 2 <= M <= 8 and (gs % 128 == 0 or K >= (2560 if M <= 5 else 3072)) else "generic"
 
 
 # ------------------------------------------------------------------ fp32 activations
@@ -102,8 +103,8 @@ def test_fp32_streaming_activation_ranges(hip, dist, bits, K, N):
 def test_fp32_streaming_groups_and_ragged_k(hip, gs, K, M):
     """Batch-1 and -2 fp32 with group sizes 32..256 and K not a multiple of 32 (the last
     chunk's pieces past K read as zero), bias and SiLU, against the oracle: the streaming kernel
-    at batch 1; at batch 2 the batched kernel for groups of 256, the fp32 matrix-core kernel for
-    groups of 32 and 64."""
+    at batch 1; at batch 2 the batched kernel for groups of 256 and, at K = 4128, its sub-unit
+    builds for groups of 32 and 64, which the fp32 matrix-core kernel takes at the shorter K."""
     w, W64, b64, _ = make(300, K, 3, torch.float32, bias=True, gs=gs)
     x = randx(M, K, torch.float32, seed=K + M)
     assert plan(torch.float32, M, K, gs, 300, 3)[0] == fp32_family(M, K, gs)

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 import cabi
-from crispybits_kernels import PackedLinearWeight, fused_gate_up, fused_qkv, packed_linear
+from crispybits_kernels import PackedLinearWeight, _C, fused_gate_up, fused_qkv, packed_linear, permute_for_rope
 from crispybits_kernels.io import from_packed_dict
 from crispybits_kernels.reference import pack_linear_dict
 from oracle import emulator as E
@@ -54,18 +54,63 @@ def test_fine_groups(hip, dtype, M, bits, N, K, gs):
         assert torch.equal(packed_linear(x, w, split_k, act="silu"), y)
 
 
-@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("gs", [32, 64])
-def test_fine_groups_fused(hip, dtype, gs):
-    M, K = 6, 1056
+def plan(dtype, M, K, gs, out, bits, kind="gemv"):
+    """Kernel family and K splits of a decode call."""
+    return _C.decode_plan(dtype, M, K, gs, out, bits, kind, 1, 1)[:2]
+
+
+@pytest.mark.parametrize("dtype,M,K,gs,N,family", [
+    (torch.float16, 3, 1024, 64, 2064, "bstream"), (torch.float16, 3, 1016, 64, 2064, "generic"),
+    (torch.float16, 10, 2560, 32, 2048, "bstream"), (torch.float16, 10, 2552, 32, 2048, "generic"),
+    (torch.bfloat16, 16, 1024, 96, 4112, "bstream"), (torch.bfloat16, 16, 3072, 64, 4096, "bstream"),
+    (torch.bfloat16, 16, 3064, 64, 4096, "generic"), (torch.float32, 2, 1536, 64, 2064, "bstream"),
+    (torch.float32, 2, 1528, 64, 2064, "generic"), (torch.float32, 8, 3072, 32, 11008, "bstream"),
+    (torch.float32, 8, 3064, 32, 11008, "generic"), (torch.float32, 9, 4096, 32, 11008, "generic"),
+    (torch.float16, 5, 4097, 64, 4096, "generic")])
+def test_fine_groups_line(hip, dtype, M, K, gs, N, family):
+    """Both sides of the line between the sub-unit builds and the fp32 matrix-core kernel."""
+    assert plan(dtype, M, K, gs, N, 4)[0] == family
+
+
+@pytest.mark.parametrize("dtype,M", [(torch.float16, 6), (torch.bfloat16, 16), (torch.float32, 2), (torch.float32, 8)])
+@pytest.mark.parametrize("gs,K", [(32, 3112), (64, 4096), (96, 11008), (64, 1056)])
+def test_fine_groups_fused(hip, dtype, M, gs, K):
+    """Fused QKV (a width per projection and one for all, with and without RoPE) and gate-up on the
+    sub-unit builds, their splits combined in the dispatch; at K = 1056 on the fp32 matrix-core kernel."""
     x = randx(M, K, dtype)
     xd = x.double().cpu().numpy()
-    ws = [make(n, K, b, dtype, gs, i) for i, (n, b) in enumerate(((1024, 4), (512, 2), (512, 3)))]
-    for o, (_, W, _) in zip(fused_qkv(x, *(w[0] for w in ws)), ws):
-        assert off(o, xd @ W.T) < BAR[dtype]
+    hd = 64
+    ws = [make(n, K, b, dtype, gs, i) for i, (n, b) in enumerate(((1024, 4), (512, 2), (512, 3), (512, 4), (512, 4)))]
+    ang = torch.rand(M, hd, generator=torch.Generator().manual_seed(9)) * 6.28
+    cos, sin = ang.cos().to(dtype).cuda(), ang.sin().to(dtype).cuda()
+    cd, sd = cos.double().cpu().numpy(), sin.double().cpu().numpy()
+
+    def rotated(y):
+        y = y.reshape(M, -1, hd)
+        half = np.concatenate([-y[..., hd // 2:], y[..., :hd // 2]], axis=-1)
+        return (y * cd[:, None] + half * sd[:, None]).reshape(M, -1)
+
+    family = "bstream" if K > 2048 else "generic"
+    for pick in ((0, 1, 2), (0, 3, 4)):
+        (q, Q, _), (k, KW, _), (v, V, _) = (ws[i] for i in pick)
+        bits = tuple(ws[i][0].bits for i in pick)
+        fam, splits = plan(dtype, M, K, gs, (1024, 512, 512), bits if len(set(bits)) > 1 else bits[0], "qkv")
+        assert fam == family and (splits > 1 or family == "generic")
+        refs = [xd @ w.T for w in (Q, KW, V)]
+        for o, ref in zip(fused_qkv(x, q, k, v), refs):
+            assert off(o, ref) < BAR[dtype]
+        refs[:2] = [rotated(y) for y in refs[:2]]
+        qp, kp = permute_for_rope(q, hd), permute_for_rope(k, hd)
+        outs = fused_qkv(x, qp, kp, v, rope=(cos, sin, hd))
+        for o, ref in zip(outs, refs):
+            assert off(o, ref) < BAR[dtype]
+        assert all(torch.equal(a, b) for a, b in zip(fused_qkv(x, qp, kp, v, rope=(cos, sin, hd)), outs))
     g, G, _ = make(1001, K, 3, dtype, gs, 5, fractional=True)
     u, U, _ = make(1001, K, 3, dtype, gs, 6, fractional=True)
-    assert off(fused_gate_up(x, g, u), E.silu64(xd @ G.T) * (xd @ U.T)) < BAR[dtype]
+    assert plan(dtype, M, K, gs, 1001, 3, "gate_up")[0] == family
+    y = fused_gate_up(x, g, u)
+    assert off(y, E.silu64(xd @ G.T) * (xd @ U.T)) < BAR[dtype]
+    assert torch.equal(fused_gate_up(x, g, u), y)
 
 
 def test_fine_groups_at_the_scratch_limit(hip):
