@@ -173,6 +173,10 @@ int cbk_packed_gemm(const void* x, int dtype, int64_t M, int64_t K,
  * elements `partial` must hold (0: the call needs none; gate_up: the gate-up GEMM's).  A call
  * without a large enough buffer runs unsplit: same result up to the order of the fp32 sums. */
 int64_t cbk_gemm_partial_floats(int dtype, int64_t M, int64_t N, int64_t K, int gate_up);
+/* The tiles of such a call with its buffer, without launching it: out[3] = {rows of a tile
+ * (32, 64 or 128), K splits, tiles}.  mode: CBK_MODE_GEMV the plain GEMM, CBK_MODE_GATEUP, or
+ * CBK_MODE_QKV (n1 and n2 are read for it only). */
+int cbk_gemm_plan(int64_t M, int64_t n0, int64_t n1, int64_t n2, int64_t K, int mode, int32_t* out);
 int cbk_packed_gemm_ws(const void* x, int dtype, int64_t M, int64_t K,
                        const int32_t* packed, const void* scales, const void* zeros, const void* bias,
                        int64_t N, int bits, int group_size, int act, int use_matrix_cores,

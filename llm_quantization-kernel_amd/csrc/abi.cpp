@@ -986,6 +986,22 @@ int cbk_packed_gemm(const void* x, int dtype, int64_t M, int64_t K, const int32_
                               use_matrix_cores, nullptr, 0, out, device, stream);
 }
 
+int cbk_gemm_plan(int64_t M, int64_t n0, int64_t n1, int64_t n2, int64_t K, int mode, int32_t* out) {
+    if (!out || M <= 0 || K <= 0 || n0 <= 0) return fail(CBK_EINVAL, "gemm_plan: sizes must be positive");
+    if (mode != CBK_MODE_GEMV && mode != CBK_MODE_QKV && mode != CBK_MODE_GATEUP)
+        return fail(CBK_EINVAL, "gemm_plan: unknown mode");
+    int64_t nt = gemm_f16_ntiles(n0, mode == CBK_MODE_GATEUP);
+    if (mode == CBK_MODE_QKV) {
+        if (n1 <= 0 || n2 <= 0) return fail(CBK_EINVAL, "gemm_plan: sizes must be positive");
+        nt += gemm_f16_ntiles(n1, false) + gemm_f16_ntiles(n2, false);
+    }
+    const GemmPlan p = gemm_f16_plan(M, nt, K, true);
+    out[0] = 32 * p.mb;
+    out[1] = p.S;
+    out[2] = (int32_t)std::min<int64_t>(p.tiles, INT32_MAX);
+    return CBK_OK;
+}
+
 int64_t cbk_gemm_partial_floats(int dtype, int64_t M, int64_t N, int64_t K, int gate_up) {
     if ((dtype != CBK_F16 && dtype != CBK_BF16) || M <= 0 || N <= 0 || K <= 0) return 0;
     return gemm_f16_plan(M, gemm_f16_ntiles(N, gate_up != 0), K, true).partial_floats;

@@ -36,6 +36,7 @@ SIGS = {
                                  _P, _P, _P, _P, _L, _P, _P, _P, _P, _L, _P, _P, _P, _P, _L,
                                  _P, _P, _I, _I, _I, _I, _I, _I, _P, _L, _P, _P, _P, _I, _P]),
     "cbk_gemm_partial_floats": (_L, [_I, _L, _L, _L, _I]),
+    "cbk_gemm_plan": (_I, [_L, _L, _L, _L, _L, _I, _P]),
     "cbk_packed_gemm_ws": (_I, [_P, _I, _L, _L, _P, _P, _P, _P, _L, _I, _I, _I, _I, _P, _L, _P, _I, _P]),
     "cbk_packed_gemm_gate_up_ws": (_I, [_P, _I, _L, _L, _P, _P, _P, _P, _P, _P, _L, _I, _I, _P, _L, _P, _I, _P]),
     "cbk_packed_gemm_gate_up": (_I, [_P, _I, _L, _L, _P, _P, _P, _P, _P, _P, _L, _I, _I, _P, _I, _P]),

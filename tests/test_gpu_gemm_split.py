@@ -1,5 +1,5 @@
-"""The 16-bit prefill GEMM below a full chip: 32- and 64-row tiles, and K split over workgroups
-whose partial tiles are combined in the dispatch.
+"""The 16-bit prefill GEMM below a full chip: 32-row tiles with K split over workgroups whose
+partial tiles are combined in the dispatch (test_gpu_gemm_tiles.py has the higher tiles).
 
 The shapes have few tiles, so that the plan splits K (cbk_gemm_partial_floats > 0 says so), with
 splits that start inside a scale window, a ragged K in the last split, partial tiles in M and N, and
