@@ -256,7 +256,21 @@ struct Group {
     bool a_tail, sz_on;              // activations: the partial last stage; whether the window is loaded
 };
 
-template <int BITS, int MB, bool TAIL, bool EVEN, bool FIRST = false>
+// Where a block's window comes from: any group size and groups of 128 codes by Sched's count of
+// blocks (the latter read their scales at lane-independent offsets), or, a window of groups of 128
+// being four blocks, from the block's index.  The same windows either way.  The index (WIN_INDEX)
+// is for the unsplit 128-row builds whose loop LLVM schedules no worse with it, by 21 shapes each
+// (plain and gate-up, batch 128 .. 2048; time against the count's in the geometric mean): fp16 W2
+// 0.98, bf16 W2 1.00, bf16 W3 0.97, fp16 W4 0.98; fp16 W3 would be 1.02, bf16 W4 1.01.  No build
+// reloads a spilled register inside the loop, so it is the order of the instructions alone.
+enum { WIN_ANY, WIN_COUNT, WIN_INDEX };
+template <int BITS, bool GS128, int DT, int MODE, int MB, bool SPLIT>
+constexpr int WINDOWS = !GS128                                     ? WIN_ANY
+                        : MB < 4 || SPLIT || MODE == GEMM_QKV      ? WIN_COUNT
+                        : BITS == 2 || (BITS == 3) == (DT == DT_BF16) ? WIN_INDEX
+                                                                   : WIN_COUNT;
+
+template <int BITS, int MB, bool TAIL, int WIN, bool EVEN, bool FIRST = false>
 __device__ __forceinline__ void group_at(const Loads<BITS, MB>& L, Sched& sc, int t, Group& g) {
     const int sa = min(t + 2, sc.nst - 1);
     g.a_tail = TAIL && sa == sc.last;
@@ -267,6 +281,12 @@ __device__ __forceinline__ void group_at(const Loads<BITS, MB>& L, Sched& sc, in
         const int j = t / 2 + 1;
         g.w_odd = j & 1;
         g.w_soff = min(j, sc.nblk - 1) * (32 * BITS);
+        if constexpr (WIN == WIN_INDEX) {
+            g.sz_on = FIRST || (j & 3) == 0;
+            g.sz_dst = g.sz_on ? L.sz_lds + ((j >> 2) & 1) * SZ_BUF : Lay<BITS, MB>::SPARE;
+            g.sz_soff = 2 * SZG * (j >> 2);
+            return;
+        }
         g.sz_on = FIRST || sc.blk_in_win == 0;
         g.sz_dst = g.sz_on ? L.sz_lds + (sc.win & 1) * SZ_BUF : Lay<BITS, MB>::SPARE;
         g.sz_soff = 2 * SZG * sc.win;
@@ -565,7 +585,7 @@ struct Ctx {
 // slots 0 .. 3 (activation stage s + 3 into the slot of stage s), read steps 0 and
 // 1 of stage s + 1 and its chunk (wn), and dequantize its step 0, leaving the entry
 // state of stage s + 1.  The last stage (!NEXT) issues nothing.  ODD: s is odd.
-template <int BITS, int MB, bool TAIL, bool GS128, int DQ, bool NEXT, bool ODD>
+template <int BITS, int MB, bool TAIL, int WIN, int DQ, bool NEXT, bool ODD>
 __device__ __forceinline__ void run_stage(Ctx<BITS, MB>& c, int s, u4 (&a)[4][MB], u4& bw, const WStage<BITS>& wc,
                                           WStage<BITS>& wn, const Group& gc, Group& gn, f16x (&acc)[MB]) {
     const int nslot = c.cslot == NST - 1 ? 0 : c.cslot + 1;
@@ -573,7 +593,7 @@ __device__ __forceinline__ void run_stage(Ctx<BITS, MB>& c, int s, u4 (&a)[4][MB
     for (int kq = 0; kq < KSTEPS; ++kq) {
         if (kq + 2 < KSTEPS) read_a<MB>(c.lds, c.cslot, kq + 2, c.ci, a[(kq + 2) & 3]);
         else if (NEXT) read_a<MB>(c.lds, nslot, kq - 2, c.ci, a[(kq + 2) & 3]);
-        if (NEXT && kq == 2) read_w<BITS, MB, GS128>(c.A, c.lds, s + 1, c.ci, wn);
+        if (NEXT && kq == 2) read_w<BITS, MB, WIN != WIN_ANY>(c.A, c.lds, s + 1, c.ci, wn);
         u4 bwn = bw;
         if (kq + 1 < KSTEPS) bwn = dequant_octet<BITS, DQ>(wc, kq + 1, c.g);
         else if (NEXT) bwn = dequant_octet<BITS, DQ>(wn, 0, c.g);
@@ -586,7 +606,7 @@ __device__ __forceinline__ void run_stage(Ctx<BITS, MB>& c, int s, u4 (&a)[4][MB
         if (NEXT && kq == 1) {
             wait_group<BITS, MB, !ODD>();             // group s (parity of s) may stay in flight
             barrier_lds();                        // stage s + 1 published
-            group_at<BITS, MB, TAIL, ODD>(c.L, c.sc, s + 1, gn);
+            group_at<BITS, MB, TAIL, WIN, ODD>(c.L, c.sc, s + 1, gn);
         }
         if (NEXT && kq >= 2) {
             issue_slot<BITS, MB, TAIL, ODD>(c.L, gn, 2 * (kq - 2), c.lds);
@@ -599,24 +619,24 @@ __device__ __forceinline__ void run_stage(Ctx<BITS, MB>& c, int s, u4 (&a)[4][MB
 // The stages, unrolled by two so the chunk and group registers of stage s and
 // stage s + 1 alternate without copies and the load-group parity is static; the
 // last stage is peeled.
-template <int BITS, int MB, bool TAIL, bool GS128, int DQ>
+template <int BITS, int MB, bool TAIL, int WIN, int DQ>
 __device__ __forceinline__ void compute_loop(Ctx<BITS, MB>& c, int s, int nst, Group& g0, f16x (&acc)[MB]) {
     u4 a[4][MB], bw;
     WStage<BITS> w0, w1;
     Group g1;
     read_a<MB>(c.lds, 0, 0, c.ci, a[0]);
     read_a<MB>(c.lds, 0, 1, c.ci, a[1]);
-    read_w<BITS, MB, GS128>(c.A, c.lds, s, c.ci, w0);
+    read_w<BITS, MB, WIN != WIN_ANY>(c.A, c.lds, s, c.ci, w0);
     bw = dequant_octet<BITS, DQ>(w0, 0, c.g);
     for (; s + 2 < nst; s += 2) {
-        run_stage<BITS, MB, TAIL, GS128, DQ, true, false>(c, s, a, bw, w0, w1, g0, g1, acc);
-        run_stage<BITS, MB, TAIL, GS128, DQ, true, true>(c, s + 1, a, bw, w1, w0, g1, g0, acc);
+        run_stage<BITS, MB, TAIL, WIN, DQ, true, false>(c, s, a, bw, w0, w1, g0, g1, acc);
+        run_stage<BITS, MB, TAIL, WIN, DQ, true, true>(c, s + 1, a, bw, w1, w0, g1, g0, acc);
     }
     if (s + 1 < nst) {
-        run_stage<BITS, MB, TAIL, GS128, DQ, true, false>(c, s, a, bw, w0, w1, g0, g1, acc);
-        run_stage<BITS, MB, TAIL, GS128, DQ, false, true>(c, s + 1, a, bw, w1, w0, g1, g0, acc);
+        run_stage<BITS, MB, TAIL, WIN, DQ, true, false>(c, s, a, bw, w0, w1, g0, g1, acc);
+        run_stage<BITS, MB, TAIL, WIN, DQ, false, true>(c, s + 1, a, bw, w1, w0, g1, g0, acc);
     } else {
-        run_stage<BITS, MB, TAIL, GS128, DQ, false, false>(c, s, a, bw, w0, w1, g0, g1, acc);
+        run_stage<BITS, MB, TAIL, WIN, DQ, false, false>(c, s, a, bw, w0, w1, g0, g1, acc);
     }
 }
 
@@ -786,6 +806,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& A, int local, int tile
     using Y = Lay<BITS, MB>;
     constexpr bool GU = MODE == GEMM_GATEUP;
     constexpr int BM = Y::BM, A_Q = Y::A_Q, SUM_IMG = Y::SUM_IMG;
+    constexpr int WIN = WINDOWS<BITS, GS128, DT, MODE, MB, SPLIT>;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int slab = wave & 3, kh = wave >> 2;    // column slab, k half of every stage
@@ -815,10 +836,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& A, int local, int tile
     sc.win = s0 / WBLK / sc.rp;
     sc.blk_in_win = s0 / WBLK - sc.win * sc.rp;
     Group g0;
-    group_at<BITS, MB, TAIL, true, true>(L, sc, s0 - 2, g0);    // stage s0, its block and window
+    group_at<BITS, MB, TAIL, WIN, true, true>(L, sc, s0 - 2, g0);    // stage s0, its block and window
 #pragma unroll
     for (int k = 0; k < SLOTS; ++k) issue_slot<BITS, MB, TAIL, true>(L, g0, k, lds);
-    group_at<BITS, MB, TAIL, false>(L, sc, s0 - 1, g0);         // stage s0 + 1
+    group_at<BITS, MB, TAIL, WIN, false>(L, sc, s0 - 1, g0);         // stage s0 + 1
 #pragma unroll
     for (int k = 0; k < A_Q; ++k) issue_slot<BITS, MB, TAIL, false>(L, g0, k, lds);
 
@@ -849,14 +870,14 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& A, int local, int tile
 
     wait_group<BITS, MB, false>();                // the first block, window and stage landed
     barrier_lds();                                // barrier s0: published
-    group_at<BITS, MB, TAIL, true>(L, sc, s0, g0);
+    group_at<BITS, MB, TAIL, WIN, true>(L, sc, s0, g0);
 #pragma unroll
     for (int k = 0; k < 4; ++k) issue_slot<BITS, MB, TAIL, true>(L, g0, k, lds);
 
     Ctx<BITS, MB> c{A, lds, ci, magic_vreg(), L, sc, 0};
     constexpr int DQ0 = DT == DT_BF16 ? 2 : 0;
-    if (fast) compute_loop<BITS, MB, TAIL, GS128, DQ0 + 1>(c, s0, nst, g0, acc);
-    else compute_loop<BITS, MB, TAIL, GS128, DQ0>(c, s0, nst, g0, acc);
+    if (fast) compute_loop<BITS, MB, TAIL, WIN, DQ0 + 1>(c, s0, nst, g0, acc);
+    else compute_loop<BITS, MB, TAIL, WIN, DQ0>(c, s0, nst, g0, acc);
     vmcnt<0>();                                   // the surplus loads land before the LDS is reused
 
     // both k halves write their partial sums row-major into a tile image of their own (fp32,
