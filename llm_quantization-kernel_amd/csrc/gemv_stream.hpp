@@ -580,13 +580,34 @@ __device__ __forceinline__ float plain_sum(const GemvArgs& A, int v, int i, int 
     return acc;
 }
 
-// The kernel's arguments read anew (GemvArgs is the batched kernel's only one), by a pointer the
-// compiler cannot see through: what only a rare path reads is then not held in registers for it (72
-// SGPRs instead of 65 in the plain W4 build), or loaded at the kernel's start.
-__device__ __forceinline__ const GemvArgs& args_again() {
-    const void* p = (const void*)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(p));
-    return *reinterpret_cast<const GemvArgs*>(p);
+// The wave's sums that are not finite formed again, in place in the workgroup's row totals.  All of
+// it comes from the kernel's arguments (GemvArgs is the batched kernel's only one), the thread and
+// the workgroup, read anew behind empty asm that the compiler cannot see through: what only this
+// rare path reads is then not held in registers through the kernel for it (held, the W2 gate-up
+// build went from 79 to 83 VGPRs, a wave fewer per SIMD, and g = 32 4096 -> 7168 at batch 3 from
+// 16.1 to 19.9 us).
+template <int BITS, int MODE, int BSU, int DT, int SUB>
+__device__ __forceinline__ void resum(char* lds) {
+    constexpr int OPR = DT == DT_F32 ? 2 : 1, NR = 4 / OPR;
+    const void* ap = (const void*)__builtin_amdgcn_kernarg_segment_ptr();
+    int tid = threadIdx.x, bx = blockIdx.x;
+    asm volatile("" : "+s"(ap), "+s"(bx), "+v"(tid));
+    const GemvArgs& A = *reinterpret_cast<const GemvArgs*>(ap);
+    const int M = A.M, RB = 16 * A.st_rw, NU = A.st_ks * BSU;
+    const int wave = tid >> 6, j = tid & 15, kq = (tid & 63) >> 4;
+    const int ks = (int)fdiv((uint32_t)wave, A.divRW), rw = wave - ks * A.st_rw;
+    const int blk = (int)fdiv((uint32_t)bx, A.divP), p = bx - blk * A.P;
+    const int roff = MODE == MODE_GATEUP ? 32 * (rw >> 1) + 2 * j + (rw & 1) : 16 * rw + j;
+    const int v = blk * RB + roff;
+    const int U = (A.C + 3) >> 2;
+    const int u0 = (int)fdiv((uint32_t)(U * p), A.divP), u1 = (int)fdiv((uint32_t)(U * (p + 1)), A.divP);
+    const int ca = 4 * (u0 + BSU * ks), cb = min(min(4 * u1, A.C), ca + 4 * BSU);
+    float* red = reinterpret_cast<float*>(lds + 256 * NU * M * OPR) + (32 * SUB + (DT != DT_F16 ? 16 : 0)) * NU;
+#pragma unroll 1
+    for (int i = NR * kq; v < A.V && i < min(NR * kq + NR, M); ++i) {
+        float* at = red + (ks * M + i) * RB + roff;
+        if (!__builtin_isfinite(*at)) *at = plain_sum<BITS, MODE, DT>(A, v, i, ca, cb);
+    }
 }
 
 template <int BITS, int MODE, int BSU, int DT, int SUB>
@@ -830,17 +851,8 @@ __device__ __forceinline__ void bstream_body(const GemvArgs& A, char* lds) {
     }
     if constexpr (SUB > 1) {
         // a sum that is not finite (infinities and NaNs in the inputs leave no other) is formed again
-        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!__builtin_isfinite(mag)) != 0, 0)) {
-            const GemvArgs& B = args_again();
-            const int bu0 = (int)fdiv((uint32_t)(((B.C + 3) >> 2) * p), B.divP);
-            const int bu1 = (int)fdiv((uint32_t)(((B.C + 3) >> 2) * (p + 1)), B.divP);
-            const int ca = 4 * (bu0 + BSU * ks), cb = min(min(4 * bu1, B.C), ca + 4 * BSU);
-#pragma unroll 1
-            for (int i = NR * kq; vin && i < min(NR * kq + NR, M); ++i) {
-                float* at = red + (ks * M + i) * RB + roff;
-                if (!__builtin_isfinite(*at)) *at = plain_sum<BITS, MODE, DT>(B, vrow, i, ca, cb);
-            }
-        }
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!__builtin_isfinite(mag)) != 0, 0))
+            resum<BITS, MODE, BSU, DT, SUB>(lds);
     }
     lds_barrier();
 }
@@ -882,12 +894,8 @@ __device__ __forceinline__ void bstream_tail(const GemvArgs& A, char* lds) {
         split_finish<DT, MODE>(A, vbase, RB, nthr);
 }
 
-// bf16 and fp32 with 8-unit slices: 768 threads at most, so 170 VGPRs (the per-unit
-// prescale does not fit 128 next to eight units of streamed chunks); the planner keeps such
-// workgroups to 12 waves.
 template <int MODE, int BITS, int BSU, int DT, int SUB>
-__global__ void __launch_bounds__(DT != DT_F16 && BSU == 8 ? 768 : 1024) gemv_bstream_kernel(const GemvArgs A) {
-    extern __shared__ __attribute__((aligned(16))) char lds[];
+__device__ __forceinline__ void bstream_job(const GemvArgs& A, char* lds) {
     if constexpr (BITS != 0) {
         bstream_body<BITS, MODE, BSU, DT, SUB>(A, lds);
     } else {
@@ -899,6 +907,36 @@ __global__ void __launch_bounds__(DT != DT_F16 && BSU == 8 ? 768 : 1024) gemv_bs
         else bstream_body<4, MODE, BSU, DT, SUB>(A, lds);
     }
     bstream_tail<MODE, BSU, DT, SUB>(A, lds);
+}
+
+// bf16 and fp32 with 8-unit slices: 768 threads at most, so 170 VGPRs (the per-unit
+// prescale does not fit 128 next to eight units of streamed chunks); the planner keeps such
+// workgroups to 12 waves.
+template <int MODE, int BITS, int BSU, int DT>
+__global__ void __launch_bounds__(DT != DT_F16 && BSU == 8 ? 768 : 1024) gemv_bstream_kernel(const GemvArgs A) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    bstream_job<MODE, BITS, BSU, DT, 1>(A, lds);
+}
+
+// The sub-unit builds.  W2 in the fused modes fits 80 VGPRs, six waves per SIMD, which LLVM misses
+// by one to five registers if it is not asked for them (W2 gate-up g = 32 fp16 batch 3 2560 -> 7168:
+// 16.1 us with six waves, 19.9 with five); likewise the mixed-width QKV build in bf16 at g = 32 and
+// 96 VGPRs.
+template <int MODE, int BITS, int DT, int SUB>
+constexpr int BSUB_WAVES = BITS == 2 && MODE != MODE_GEMV && (DT == DT_F16 || (DT == DT_BF16 && SUB == 2)) ? 6
+                           : BITS == 0 && DT == DT_BF16 && SUB == 4                                       ? 5
+                                                                                                          : 4;
+template <int MODE, int BITS, int BSU, int DT, int SUB>
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(BSUB_WAVES<MODE, BITS, DT, SUB>)))
+gemv_bsub_kernel(const GemvArgs A) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    bstream_job<MODE, BITS, BSU, DT, SUB>(A, lds);
+}
+
+template <int MODE, int BITS, int BSU, int DT, int SUB>
+const void* bstream_entry() {
+    if constexpr (SUB == 1) return reinterpret_cast<const void*>(&gemv_bstream_kernel<MODE, BITS, BSU, DT>);
+    else return reinterpret_cast<const void*>(&gemv_bsub_kernel<MODE, BITS, BSU, DT, SUB>);
 }
 
 // BITS = 0: fused QKV with a width per projection; the host keeps each
@@ -925,11 +963,10 @@ __global__ void __launch_bounds__(1024) gemv_stream_kernel(const GemvArgs A) {
 
 template <int BSU, int DT, int SUB>
 const void* bstream_kernel(int mode, int bits, bool mixed) {
-    if (mixed) return reinterpret_cast<const void*>(&gemv_bstream_kernel<MODE_QKV, 0, BSU, DT, SUB>);
-#define CBK_BSTREAM_K(M)                                                                                \
-    (bits == 2 ? reinterpret_cast<const void*>(&gemv_bstream_kernel<M, 2, BSU, DT, SUB>)                \
-               : (bits == 3 ? reinterpret_cast<const void*>(&gemv_bstream_kernel<M, 3, BSU, DT, SUB>)   \
-                            : reinterpret_cast<const void*>(&gemv_bstream_kernel<M, 4, BSU, DT, SUB>)))
+    if (mixed) return bstream_entry<MODE_QKV, 0, BSU, DT, SUB>();
+#define CBK_BSTREAM_K(M)                                      \
+    (bits == 2 ? bstream_entry<M, 2, BSU, DT, SUB>()          \
+               : (bits == 3 ? bstream_entry<M, 3, BSU, DT, SUB>() : bstream_entry<M, 4, BSU, DT, SUB>()))
     if (mode == MODE_QKV) return CBK_BSTREAM_K(MODE_QKV);
     if (mode == MODE_GATEUP) return CBK_BSTREAM_K(MODE_GATEUP);
     return CBK_BSTREAM_K(MODE_GEMV);
