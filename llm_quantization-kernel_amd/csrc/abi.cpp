@@ -456,25 +456,29 @@ bool bstream_fills(const BStreamPlan& base, int64_t V) {
     return base.P > 1 || ceil_div(V, 16 * base.rw) * base.P * 2 <= BSTREAM_CU_TARGET;
 }
 
-// The shortest K at which a call with groups finer than a unit leaves the fp32 matrix-core kernel.
-// That kernel has no activations to stage and no splits, and its time follows K: 5 us at 512, 8 at
-// 2048, 12 at 2560, 17 at 4096 up to 4096 rows, in proportion to the rows past that.  The sub-unit
-// builds cost 4.5 .. 7 us where one split's row blocks cover half the CUs (V > 2048, or 4096 with
-// the two row groups of more than 10 operand rows), else 7 (3 operand rows) to 13 (16) for the
-// splits, hardly more with K.  So the line is low with enough rows (16-bit x; fp32 x at batch 2
-// stages more) and otherwise lies where the other kernel passes the splits' cost.  Measured over
-// 784 points (K 512 .. 4096, V 512 .. 14336, batch 2 .. 16, g = 32 and 64), us, that kernel / this
-// one: fp16 batch 3 V 4096 K 1024 6.2 / 4.6; V 1024 K 2048 7.6 / 7.7, K 2560 8.8 / 7.7; batch 16
-// V 4096 K 2088 8.5 / 11.2, K 3072 13.8 / 11.7; V 8192 K 1024 9.8 / 7.0, K 512 6.6 / 6.5; fp32
-// batch 8 V 8192 K 2088 14.1 / 21.5, K 3072 25.8 / 23.8.
-int bstream_fine_k(int64_t rows, int64_t V, int dtype) {
-    const bool full = V > (rows <= 10 ? 2048 : 4096);
-    if (full && dtype != CBK_F32) return 1024;
-    if (full && rows <= 4) return 1536;
-    return rows <= 10 ? 2560 : 3072;
+// Whether a call with groups finer than a unit leaves the fp32 matrix-core kernel for its streaming
+// plan (rows: operand rows; split: the plan has K splits).  That kernel has no activations to stage
+// and no splits, and its time follows K: 5 us at 512, 7 at 1280, 10 at 2560, 13 at 3584 up to 4096
+// rows, in proportion to the rows past that, and up to a third more where K is a multiple of 1024.
+// The sub-unit builds take 4.5 .. 8 us where the plan is unsplit (its row blocks cover half the CUs),
+// else 7 .. 11 for the splits, hardly more with K.  So the line is low for unsplit plans (higher for
+// fp32, which stages two operand rows a row) and else lies where the other kernel passes the splits'
+// cost.  Groups other than 32 and multiples of 64 (96, 160) cost that kernel less, and these builds,
+// with their sub-units of 32, no less.  Measured over 36792 points (K 512 .. 6144, V 512 .. 14336,
+// batch 2 .. 16, g 32, 64 and 96, every width and dtype), the rule takes 0.74 of that kernel's time in
+// the geometric mean and is slower by more than 3 % at 0.3 % of them (at worst 1.24: fp32 batch 8
+// K 4352 V 2064 g 32, whose plan is a little over one workgroup per CU).  us, that kernel / this one:
+// fp16 batch 3 g 64 V 4096 K 1024 6.8 / 4.9 unsplit; batch 10 V 2064 K 1024 6.9 / 8.9, K 2560 10.5 /
+// 9.1 (4 splits); batch 16 V 4096 K 2560 10.8 / 9.6, K 3072 15.1 / 9.8 (2); V 8192 K 1024 10.8 / 6.2.
+bool bstream_fine(int64_t rows, int64_t V, int64_t K, int gs, int dtype, bool split) {
+    const bool whole = gs % 64 == 0, odd = !whole && gs > 32;
+    if (!split)
+        return K >= (dtype == CBK_F32 ? (rows <= 4 ? 1536 : (odd ? 3072 : 2560)) : (odd && V < 8192 ? 1536 : 1024));
+    if (odd || rows > 10) return K >= 3072;
+    return (whole && V > 2048 && K % 1024 == 0 ? K + K / 4 : K) >= 2560;
 }
 
-BStreamPlan plan_bstream(const GemvArgs& A, int dtype, int mode, bool mixed, int split_k, int cus) {
+BStreamPlan plan_bstream_units(const GemvArgs& A, int dtype, int mode, bool mixed, int split_k, int cus) {
     BStreamPlan bp;
     const int64_t lim = INT32_MAX;
     // bf16 with 8-unit slices runs a 768-thread build of the kernel (its per-unit prescale
@@ -495,7 +499,6 @@ BStreamPlan plan_bstream(const GemvArgs& A, int dtype, int mode, bool mixed, int
     const bool gateup = mode == CBK_MODE_GATEUP;
     const int64_t U = ceil_div(A.C, 4);
     const int sub = bstream_sub(A.gs);
-    if (sub > 1 && A.K < bstream_fine_k(A.M * xr, A.V, dtype)) return bp;
     bp = bstream_base(A.M, A.C, split_k, gateup, bf, xr, sub);
     if (bstream_fills(bp, A.V)) {
         BStreamPlan fill = bstream_fill(A, mode, mixed, std::max(split_k, 1), bf, xr, sub);
@@ -527,6 +530,12 @@ BStreamPlan plan_bstream(const GemvArgs& A, int dtype, int mode, bool mixed, int
         }
     }
     return bstream_make(A, mode, mixed, bp.P, bp.bsu, bp.rw, bf, xr, sub);
+}
+
+BStreamPlan plan_bstream(const GemvArgs& A, int dtype, int mode, bool mixed, int split_k, int cus) {
+    const BStreamPlan bp = plan_bstream_units(A, dtype, mode, mixed, split_k, cus);
+    const int64_t rows = (int64_t)A.M * (dtype == CBK_F32 ? 2 : 1);
+    return bp.ok && bp.sub > 1 && !bstream_fine(rows, A.V, A.K, A.gs, dtype, bp.P > 1) ? BStreamPlan() : bp;
 }
 
 // Kernels (per device) whose dynamic-LDS limit has been raised to the whole budget.  The

@@ -62,14 +62,18 @@ def plan(dtype, M, K, gs, out, bits, kind="gemv"):
 @pytest.mark.parametrize("dtype,M,K,gs,N,family", [
     (torch.float16, 3, 1024, 64, 2064, "bstream"), (torch.float16, 3, 1016, 64, 2064, "generic"),
     (torch.float16, 10, 2560, 32, 2048, "bstream"), (torch.float16, 10, 2552, 32, 2048, "generic"),
-    (torch.bfloat16, 16, 1024, 96, 4112, "bstream"), (torch.bfloat16, 16, 3072, 64, 4096, "bstream"),
-    (torch.bfloat16, 16, 3064, 64, 4096, "generic"), (torch.float32, 2, 1536, 64, 2064, "bstream"),
-    (torch.float32, 2, 1528, 64, 2064, "generic"), (torch.float32, 8, 3072, 32, 11008, "bstream"),
-    (torch.float32, 8, 3064, 32, 11008, "generic"), (torch.float32, 9, 4096, 32, 11008, "generic"),
-    (torch.float16, 5, 4097, 64, 4096, "generic")])
+    (torch.float16, 9, 2048, 64, 2064, "bstream"), (torch.float16, 9, 1024, 64, 3072, "generic"),
+    (torch.bfloat16, 16, 1024, 32, 4112, "bstream"), (torch.bfloat16, 16, 1024, 96, 4112, "generic"),
+    (torch.bfloat16, 16, 3072, 64, 4096, "bstream"), (torch.bfloat16, 16, 3064, 64, 4096, "generic"),
+    (torch.float32, 2, 1536, 64, 2064, "bstream"), (torch.float32, 2, 1528, 64, 2064, "generic"),
+    (torch.float32, 8, 2560, 32, 11008, "bstream"), (torch.float32, 8, 2552, 32, 11008, "generic"),
+    (torch.float32, 9, 4096, 32, 11008, "generic"), (torch.float16, 5, 4097, 64, 4096, "generic")])
 def test_fine_groups_line(hip, dtype, M, K, gs, N, family):
-    """Both sides of the line between the sub-unit builds and the fp32 matrix-core kernel."""
+    """Both sides of the line between the sub-unit builds and the fp32 matrix-core kernel: low where
+    the streaming plan has no splits, which batch 9 and 10 with V <= 4096 rows, or gate-up there, do."""
     assert plan(dtype, M, K, gs, N, 4)[0] == family
+    if K == 1024 and N < 4096:
+        assert plan(dtype, M, K, gs, N // 2, 4, "gate_up")[0] == "generic"
 
 
 @pytest.mark.parametrize("dtype,M", [(torch.float16, 6), (torch.bfloat16, 16), (torch.float32, 2), (torch.float32, 8)])
@@ -222,6 +226,7 @@ def test_fine_groups_not_finite(hip, dtype, kind, gs, M, K):
             t[17, 0] = float("inf")
     off1 = torch.empty(M * K + 1, dtype=dtype, device="cuda")[1:].view(M, K).copy_(x)
     bar = BAR[dtype]
+    assert plan(dtype, M, K, gs, 1024, 4)[0] == "bstream"
     y, z = packed_linear(x, ws[0]), packed_linear(off1, ws[0])
     same_specials(y, z, bar)
     assert z.isinf().any() or kind != "x inf"
