@@ -184,7 +184,8 @@ int cbk_packed_gemm_ws(const void* x, int dtype, int64_t M, int64_t K,
 
 /* Prefill gate-up: out[M,N] = RN_T(RN_T(silu(x . G-hat^T)) * RN_T(x . U-hat^T)) in one launch,
  * bit-identical to two cbk_packed_gemm calls (the gate's with act = 2) followed by an
- * elementwise product in T.  No counterpart in the reference's _C: it replaces the
+ * elementwise product in T.  (The _ws calls may split K, each by its own plan: then the order
+ * of the fp32 sums differs.)  No counterpart in the reference's _C: it replaces the
  * two-GEMM-and-multiply sequence of the reference's ops.fused_gate_up for batches above the
  * decode threshold (Kernel/crispybits_kernels/ops.py:216-220).  fp16 / bf16 x only, with
  * K % 8 == 0 and 16-byte aligned x, packed, scales and zeros; other calls return

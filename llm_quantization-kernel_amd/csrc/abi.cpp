@@ -320,9 +320,9 @@ StreamPlan plan_stream(const GemvArgs& A, int dtype, int mode, bool mixed, int s
     return sp;
 }
 
-// Batched streaming plan (gemv_stream.hip, bstream), batch 3..16 for fp16 or bf16 x and
-// 2..8 for fp32 x, with 16-byte pieces, group sizes that are multiples of 128 (a unit of 128 codes is one
-// group), 32-bit offsets, and rows that keep every 16-row tile inside one projection
+// Batched streaming plan (gemv_stream.hpp, bstream), batch 3..16 for fp16 or bf16 x and
+// 2..8 for fp32 x, with 16-byte pieces, any group size (a unit of 128 codes lies in one group, or
+// has sub-units that do: slices of 4 units then, and bstream_fine), 32-bit offsets, and rows that keep every 16-row tile inside one projection
 // (fused QKV: Q and K widths multiples of 16; mixed widths: of the workgroup's rows).
 // K is split over units; a split's units are cut into slices of bsu units (one wave
 // each, at most 16 waves): 4 where that needs no split, else 8.  The split grows until

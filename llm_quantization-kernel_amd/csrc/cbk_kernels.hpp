@@ -25,7 +25,7 @@ constexpr int STREAM_CPL = CBK_STREAM_CPL;
 constexpr int STREAM_RPW = 4;
 constexpr int STREAM_RPW_WIDE = 8;
 const void* gemv_stream_kernel_for(int mode, int bits, bool mixed, int mb, int rpw, int dt);
-// gemv_stream.hip: batch 3..16, fp16 or bf16, group size % 128 == 0 (sub 1).  A job is 16 * st_rw virtual
+// gemv_stream.hip: batch 3..16, fp16 or bf16 (fp32: 2..8), group size % 128 == 0 (sub 1).  A job is 16 * st_rw virtual
 // rows x one K split (over 128-code units); its workgroup has st_ks * st_rw waves, each
 // over 16 rows and one K slice of bsu (4 or 8) units.
 const void* gemv_bstream_kernel_for(int mode, int bits, bool mixed, int bsu, int dt, int sub);
@@ -85,7 +85,7 @@ hipError_t launch_gemm_mfma(const GemmArgs& A, int dt, hipStream_t stream);
 // gemm_f32.hip: any dtype, fp32 operands on the fp32 matrix cores, W-hat unrounded.
 hipError_t launch_gemm_f32(const GemmArgs& A, int dt, hipStream_t stream);
 
-// gemm_f16.hip: fp16 or bf16 (dt), K % 8 == 0, 16-byte aligned x.  gate_up: out =
+// gemm_f16.cpp: fp16 or bf16 (dt), K % 8 == 0, 16-byte aligned x.  gate_up: out =
 // silu(x . W-hat^T) * (x . W2-hat^T), each factor rounded to the dtype first (no bias).
 // A call's plan: tiles of 32 mb rows (mb 1, 2 or 4) x 128 columns, S K splits each.
 struct GemmPlan {

@@ -1,6 +1,6 @@
 // gemm.hip -- prefill packed GEMM: out[M,N] = act(x . W-hat^T + bias).
 //
-// The matrix-core prefill for fp16 / bf16 shapes gemm_f16.hip does not take (K % 8 != 0,
+// The matrix-core prefill for fp16 / bf16 shapes gemm_f16_tile.hpp does not take (K % 8 != 0,
 // x or metadata not 16-byte aligned): cb_gemm_tc_kernel's contract
 // (Kernel/csrc/packed_gemm.cu:12-115).
 //

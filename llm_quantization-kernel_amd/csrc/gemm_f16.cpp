@@ -29,8 +29,8 @@ bool gemm_f16_supported(const GemmArgs& A) {
 // cost another round; a split adds the round trip of its partial tiles.  The constants (us) are
 // fitted to 2272 measured (shape, batch, tile, split) points: N 1024 .. 13824, K 512 .. 13824,
 // batch 17 .. 1024, W4 / W3, fp16 / bf16, plain and gate-up, on 256 CUs.  Its pick is 0.6 % off
-// the fastest point in the geometric mean, at worst 9 %, and 1.25x faster than 128-row tiles
-// unsplit, at no point slower (W4, us: 11008 -> 4096 batch 32 68.0 -> 17.5, batch 256 68.9 -> 41.0;
+// the fastest point in the geometric mean, at worst 9 %, and 1.25x faster than the same kernel's
+// 128-row tiles unsplit, at none of those points slower (W4, us: 11008 -> 4096 batch 32 68.0 -> 17.5, batch 256 68.9 -> 41.0;
 // 4096^2 batch 128 29.9 -> 18.1).
 GemmPlan gemm_f16_plan(int64_t M, int64_t ntiles, int64_t K, bool split) {
     struct Cost {

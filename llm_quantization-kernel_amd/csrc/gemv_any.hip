@@ -1,9 +1,10 @@
 // gemv_any.hip -- decode GEMV for every activation dtype, group size and row layout, on
 // the fp32 matrix cores; and the launch that combines split-K partials.
 //
-// Takes the decode calls the streaming kernels (gemv_stream.hip) do not: fp32
-// activations at any batch, fp16 / bf16 activations that are not 16-byte aligned (or
-// K % 8 != 0), group sizes 32 and 64 at batch 3..16, and batches above 16.  It keeps
+// Takes the decode calls the streaming kernels (gemv_stream.hpp) do not: fp32
+// activations above batch 8, activations that are not 16-byte aligned (or K % 8 != 0),
+// groups finer than 128 codes at batch 3..16 (fp32 2..8) and short K (bstream_fine, abi.cpp) or
+// without room for the splits of that plan, and batches above 16.  It keeps
 // the reference decode's arithmetic contract (Kernel/csrc/packed_gemv.cu:84-163): fp32
 // throughout from the T inputs, one rounding to T at the end, for the plain, fused-QKV
 // (mixed widths included) and fused gate-up modes.

@@ -169,3 +169,22 @@ def test_partial_query():
     assert lib.cbk_gemv_partial_floats(0, 16, 64, 16384, 128, 1) > 0
     # fp32 batch 8 stages 16 operand rows: K 11008 needs at least 3 splits for the LDS
     assert lib.cbk_gemv_partial_floats(2, 8, 4096, 11008, 128, 1) >= 3 * 8 * 4096
+
+
+def test_gemm_plan():
+    """The prefill plan: tile rows of 32, 64 or 128, splits only where the call has a partial buffer
+    to ask for, of tiles x splits partial tiles; bad arguments are errors."""
+    import ctypes
+    out = (ctypes.c_int32 * 3)()
+    for M in (17, 77, 256, 2048):
+        for N, K in ((256, 512), (4096, 4096), (4096, 11008), (11008, 4096)):
+            for gate_up, mode in ((0, 0), (1, 2)):
+                assert _lib().cbk_gemm_plan(M, N, 0, 0, K, mode, out) == 0
+                rows, splits, tiles = out
+                assert rows in (32, 64, 128) and splits >= 1
+                assert tiles == -(-M // rows) * -(-N // (64 if gate_up else 128))
+                floats = _lib().cbk_gemm_partial_floats(0, M, N, K, gate_up)
+                assert floats == (tiles * splits * rows * 128 if splits > 1 else 0)
+    assert _lib().cbk_gemm_plan(77, 4096, 1024, 1024, 4096, 1, out) == 0
+    for bad in ((0, 64, 0, 0, 256, 0), (8, 64, 0, 0, 256, 3), (8, 64, 0, 64, 256, 1)):
+        assert _lib().cbk_gemm_plan(*bad, out) == 1 and "gemm_plan" in _err()
